@@ -390,3 +390,27 @@ def test_timestral_forecast_covariate_errors(ta, gpu_ready):
     assert ta.timestral_forecast(out, xd, od, tm, 2, 1, x.shape[1], 40, known=kd) == ta.E_UNSUPPORTED
     assert "KnownCovariatesUnsupported" in ta.last_error()
     assert ta.timestral_forecast(out, xd, od, tm, 2, 1, x.shape[1], 40, past=pd) == ta.OK, ta.last_error()
+
+
+@pytest.mark.parametrize("length,ps,lead", [(1024, 16, 0), (1040, 16, 1030), (1023, 16, 600), (2100, 16, 1100),
+                                            (1536, 64, 700), (530, 8, 513), (900, 256, 300)])
+def test_timestral_rows_longer_than_a_tile(ta, orc, orc16, gpu_ready, length, ps, lead):
+    """The row kernels around their tile and pass edges: statistics tiles of at most 1024 steps (whole
+    patches of 8, 16, 64 and 256 steps, the state carried over the edge and over decode blocks), the
+    forward fill's 512-step passes (a first observation in a later pass, gaps across an edge), the
+    refine fold with patches wider than a wave and the cap's bounds, against both oracle builds and
+    float64 at the bar; cached decoding continues the carried statistics."""
+    rng = np.random.default_rng(length + ps)
+    b, v = 2, 2
+    m = _ref.timestral_model(rng, ps=ps, d=128, nh=2, hid=128, schedule=("time_variate",), context_length=4096)
+    t = np.arange(length)
+    x = (20 + 6 * np.sin(2 * np.pi * t / 24) + 0.02 * t + rng.standard_normal((b * v, length))).astype(np.float32)
+    obs = rng.random((b * v, length)) >= 0.1
+    obs[0, :lead] = False
+    obs[1, 500:530] = False
+    x[~obs] = 0
+    horizon = 3 * ps + ps // 2 + 1
+    got = _gpu(ta, m, x, obs, b, v, horizon, per_shot=2)
+    w8, w16 = (_oracle(o_, m, x, obs, b, v, horizon, 0, 2) for o_ in (orc, orc16))
+    assert np.isfinite(got).all()
+    _ref.assert_within_reference_bar(got, w8, w16, _ref.timestral_forecast_f64(m, x, obs, b, v, horizon, per_shot=2))

@@ -9,9 +9,11 @@
 // and known-future covariate rows (the window, the known rows' statistics and the role feedback).
 //
 // The sequential recurrences of the reference (the float64 Welford of every row, the fold of
-// refineBlock) run one thread per row in the reference's order, so they give the reference's
-// values; a row's state is kept between decode blocks and continued over the appended steps,
-// which is the same sequence of operations as recomputing the grown row from its start.
+// refineBlock) run one workgroup per row: what hangs on no earlier step (the loads, the divisions,
+// the deviations) is spread over the threads, and only the chains of additions are walked by one
+// lane, in the reference's order, so they give the reference's values; a row's state is kept
+// between decode blocks and continued over the appended steps, which is the same sequence of
+// operations as recomputing the grown row from its start.
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -29,9 +31,12 @@ __device__ __forceinline__ double fmax_d(double a, double b) { return fmax(a, b)
 // and n_known known-future covariates (NaN = missing). Keep the last `keep` steps, left-pad to t;
 // known rows also write their horizon values to kf/kfm (rows, hpad). Also the clip flag of each
 // target input row (finish, :163-178).
-__global__ void ts_context(const TsContextParams p) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= p.rows) return;
+// One workgroup per row: the forward fill of a step is the value of the last observed lane at or
+// before it (a ballot and a shuffle), else that of an earlier wave or an earlier pass over the row. One
+// thread per row walked every step behind its load (24 rows x 1500 steps: 557 us; now under 7 us).
+constexpr int kCtxT = 512;
+__global__ __launch_bounds__(kCtxT) void ts_context(const TsContextParams p) {
+    const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = r / p.vall, i = r % p.vall;
     const bool mirror = g >= p.batch;
     const int sidx = mirror ? g - p.batch : g;
@@ -39,7 +44,7 @@ __global__ void ts_context(const TsContextParams p) {
     const int t0 = p.t0, keep = p.keep, t = p.t;
     float* c = p.ctx + (int64_t)r * p.cap_t;
     uint8_t* mk = p.mask + (int64_t)r * p.cap_t;
-    for (int j = 0; j < t - keep; j++) {
+    for (int j = tid; j < t - keep; j += kCtxT) {
         c[j] = 0.f;
         mk[j] = 0;
     }
@@ -47,7 +52,7 @@ __global__ void ts_context(const TsContextParams p) {
         const bool known = i >= p.V + p.n_past;
         const float* x = known ? p.known + ((int64_t)sidx * p.n_known + (i - p.V - p.n_past)) * (t0 + p.horizon)
                                : p.past + ((int64_t)sidx * p.n_past + (i - p.V)) * t0;
-        for (int j = t0 - keep; j < t0; j++) {
+        for (int j = t0 - keep + tid; j < t0; j += kCtxT) {
             const float v = sign * x[j];
             const bool ob = !isnan(v);
             const int dst = (t - keep) + (j - (t0 - keep));
@@ -55,7 +60,7 @@ __global__ void ts_context(const TsContextParams p) {
             mk[dst] = ob ? 1 : 0;
         }
         if (known)
-            for (int j = 0; j < p.hpad; j++) {
+            for (int j = tid; j < p.hpad; j += kCtxT) {
                 const float v = j < p.horizon ? sign * x[t0 + j] : 0.f;
                 const bool ob = j < p.horizon && !isnan(v);
                 p.kf[(int64_t)r * p.hpad + j] = ob ? v : 0.f;
@@ -63,29 +68,55 @@ __global__ void ts_context(const TsContextParams p) {
             }
         return;
     }
+    constexpr int NW = kCtxT / 64;
+    __shared__ float wave_last[2][NW];  // by the pass's parity: the last observed value of each wave,
+    __shared__ int wave_seen[2][NW];    // and whether it has one
+    __shared__ int any_s, neg_s;
     const int src = sidx * p.V + i;
     const float* x = p.inputs + (int64_t)src * t0;
     const uint8_t* o = p.observed + (int64_t)src * t0;
-    float last = 0.f;
-    bool seen = false, any = false, all_nonneg = true;
-    for (int j = 0; j < t0; j++) {
-        const float v = sign * x[j];
-        const bool ob = o[j] != 0;
-        if (ob) {
-            last = v;
-            seen = true;
-            if (isfinite(x[j])) {
-                any = true;
-                all_nonneg = all_nonneg && x[j] >= 0.f;
-            }
+    if (tid == 0) any_s = neg_s = 0;
+    float last = 0.f;  // the last observed value before the pass (uniform over the workgroup)
+    bool seen = false, any = false, neg = false;
+    int par = 0;
+    for (int j0 = 0; j0 < t0; j0 += kCtxT, par ^= 1) {
+        const int j = j0 + tid;
+        const float xj = j < t0 ? x[j] : 0.f, v = sign * xj;
+        const bool ob = j < t0 && o[j] != 0;
+        if (ob && isfinite(xj)) {
+            any = true;
+            neg = neg || !(xj >= 0.f);
         }
-        if (j >= t0 - keep) {
+        const unsigned long long all = __ballot(ob), upto = all & (~0ull >> (63 - lane));
+        const float fill = __shfl(v, upto ? 63 - __clzll(upto) : lane);
+        if (lane == (all ? 63 - __clzll(all) : 0)) {
+            wave_last[par][wave] = v;
+            wave_seen[par][wave] = all != 0;
+        }
+        __syncthreads();  // (the other parity's arrays are free for the next pass)
+        float before = last;
+        bool sb = seen;
+        for (int w = 0; w < NW; w++) {
+            if (!wave_seen[par][w]) continue;
+            if (w < wave) {
+                before = wave_last[par][w];
+                sb = true;
+            }
+            last = wave_last[par][w];
+            seen = true;
+        }
+        if (j < t0 && j >= t0 - keep) {
             const int dst = (t - keep) + (j - (t0 - keep));
-            c[dst] = seen ? last : 0.f;
+            c[dst] = upto ? fill : sb ? before : 0.f;
             mk[dst] = ob ? 1 : 0;
         }
     }
-    if (!mirror) p.nonneg[src] = any && all_nonneg;
+    if (mirror) return;
+    __syncthreads();
+    if (any) any_s = 1;
+    if (neg) neg_s = 1;
+    __syncthreads();
+    if (tid == 0) p.nonneg[src] = any_s != 0 && neg_s == 0;
 }
 
 // predictBlock's window with covariates (model.zig:253-273): steps [t, t + blen) of every row are
@@ -149,7 +180,8 @@ __global__ void ts_known_stats(const float* ctx, const uint8_t* mask, int cap_t,
 }  // namespace
 
 hipError_t launch_ts_context(const TsContextParams& p, hipStream_t s) {
-    hipLaunchKernelGGL(ts_context, dim3((unsigned)((p.rows + 63) / 64)), dim3(64), 0, s, p);
+    if (p.rows <= 0) return hipSuccess;
+    hipLaunchKernelGGL(ts_context, dim3((unsigned)p.rows), dim3(kCtxT), 0, s, p);
     return hipGetLastError();
 }
 
@@ -177,72 +209,158 @@ namespace {
 // (model.zig:343-357: observed, or with attend_missing any patch after the row's first observed
 // one), the row's first observed patch (-1 if none yet), and refineBlock's fold of the context's
 // per-patch moments (forecaster.zig:613-631) into fold (w, mean, m2).
-__global__ void ts_stats(const TsStatsParams p) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= p.rows) return;
+// One workgroup per row, in tiles of whole patches held in LDS. The chains of rounded operations
+// (cum_x, m2, the fold's mean and m2) keep the reference's order, one lane each; the loads, the
+// divisions and every term that hangs on no other step are spread over the threads. One thread per
+// row did all of it behind each step's load and divisions (24 rows x 1504 steps: 337 us; now
+// 36 us, bound by the two chains of 1504 additions).
+constexpr int kStatsT = 256, kStatsTile = 1024;
+
+// c += s[i], i < n (n rounded up to 8: the padding is zeros), each partial sum to out[i].
+__device__ __forceinline__ double chain_sum(const double* s, double* out, int n, double c) {
+    for (int i0 = 0; i0 < n; i0 += 8) {
+        double v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = s[i0 + k];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            c += v[k];
+            out[i0 + k] = c;
+        }
+    }
+    return c;
+}
+
+__global__ __launch_bounds__(kStatsT) void ts_stats(const TsStatsParams p) {
+    __shared__ double sx[kStatsTile];                  // w x of each step, then its term of m2, then m2 after it
+    __shared__ double cx[kStatsTile], cw[kStatsTile];  // cum_x, cum_w after each step
+    // Per patch: observed steps, their mean (then the fold's delta), their m2, 1 / the fold's count.
+    __shared__ double pm_cnt[kStatsTile], pm_mean[kStatsTile], pm_m2[kStatsTile], pm_inv[kStatsTile];
+    __shared__ double st_s[4], fo_s[3];  // the row's state after the tile
+    __shared__ int first_s;              // first observed patch so far
+    const int r = blockIdx.x, tid = threadIdx.x;
     const float* x = p.ctx + (int64_t)r * p.cap_t;
     const uint8_t* o = p.mask + (int64_t)r * p.cap_t;
     double* st = p.state + (int64_t)r * 4;
     double* fo = p.fold + (int64_t)r * 3;
-    double cum_w = 0, cum_x = 0, m2 = 0, prev_mean = 0;
-    double fw = 0, fmean = 0, fm2 = 0;
-    int first = -1;
-    if (p.from > 0) {
-        cum_w = st[0]; cum_x = st[1]; m2 = st[2]; prev_mean = st[3];
-        fw = fo[0]; fmean = fo[1]; fm2 = fo[2];
-        first = p.row_first[r];
-    }
-    const int ps = p.ps;
-    for (int pt = p.from / ps; pt < p.t / ps; pt++) {
-        bool ob_any = false;
-        double cnt = 0, sum = 0;
-        for (int k = 0; k < ps; k++) {
-            const int i = pt * ps + k;
-            const bool ob = o[i] != 0;
-            const double w = ob ? 1.0 : 0.0;
-            const double xv = (double)x[i];
-            cum_w += w;
-            cum_x += w * xv;
-            const double den = fmax_d(cum_w, 1.0);
-            const double mean = cum_x / den;
-            m2 += (xv - prev_mean) * (xv - mean) * w;
-            prev_mean = mean;
-            if (ob) {
-                ob_any = true;
-                cnt += 1;
-                sum += (double)x[i];
+    const int ps = p.ps, pt_end = p.t / ps, per = kStatsTile / ps;  // whole patches per tile
+    if (tid < 4) st_s[tid] = p.from > 0 ? st[tid] : 0.0;
+    else if (tid < 7) fo_s[tid - 4] = p.from > 0 ? fo[tid - 4] : 0.0;
+    else if (tid == 7) first_s = p.from > 0 && p.row_first[r] >= 0 ? p.row_first[r] : 0x7fffffff;
+    __syncthreads();
+    for (int pt0 = p.from / ps; pt0 < pt_end; pt0 += per) {
+        const int np = min(per, pt_end - pt0), n = np * ps;
+        double xv[kStatsTile / kStatsT];
+#pragma unroll
+        for (int k = 0; k < kStatsTile / kStatsT; k++) {
+            const int i = tid + kStatsT * k;
+            const double w = i < n && o[pt0 * ps + i] != 0 ? 1.0 : 0.0;
+            xv[k] = i < n ? (double)x[pt0 * ps + i] : 0.0;
+            sx[i] = w * xv[k];
+            cw[i] = w;
+        }
+        const double cum_w0 = st_s[0], mean_in = st_s[3], fold_w0 = fo_s[0];
+        __syncthreads();
+        if (tid == 0) {
+            st_s[1] = chain_sum(sx, cx, n, st_s[1]);
+        } else if (tid >= 64) {
+            // The patch's own moments (forecaster.zig:613-631), each over its observed steps in order.
+            for (int q = tid - 64; q < np; q += kStatsT - 64) {
+                double cnt = 0, sum = 0, mean = 0, m2 = 0;
+                for (int k = 0; k < ps; k++)
+                    if (cw[q * ps + k] != 0) {
+                        cnt += 1;
+                        sum += sx[q * ps + k];
+                    }
+                if (cnt > 0) {
+                    mean = sum / fmax_d(cnt, 1.0);
+                    for (int k = 0; k < ps; k++)
+                        if (cw[q * ps + k] != 0) {
+                            const double dv = sx[q * ps + k] - mean;
+                            m2 += dv * dv;
+                        }
+                    atomicMin(&first_s, pt0 + q);
+                }
+                pm_cnt[q] = cnt;
+                pm_mean[q] = mean;
+                pm_m2[q] = m2;
             }
         }
-        const double den = fmax_d(cum_w, 1.0);
-        const double variance = m2 / fmax_d(den - 1.0, 1.0);
-        p.loc[(int64_t)r * p.cap_p + pt] = (float)prev_mean;
-        p.scale[(int64_t)r * p.cap_p + pt] = (float)fmax_d(sqrt(variance), p.min_scale);
-        if (ob_any && first < 0) first = pt;
-        p.key_valid[(int64_t)r * p.cap_p + pt] = (uint8_t)(p.attend_missing ? (ob_any || first >= 0) : ob_any);
-        // refineBlock's per-patch moments, combined with welfordCombine (forecaster.zig:567-577)
-        double pm_mean = 0, pm_m2 = 0;
-        if (cnt > 0) {
-            pm_mean = sum / fmax_d(cnt, 1.0);
-            for (int k = 0; k < ps; k++)
-                if (o[pt * ps + k]) {
-                    const double dv = (double)x[pt * ps + k] - pm_mean;
-                    pm_m2 += dv * dv;
+        __syncthreads();
+        if (tid < 64) {  // counts: whole numbers, the same in any order
+            double c = cum_w0;
+            for (int i0 = 0; i0 < n; i0 += 64) {
+                double v = i0 + tid < n ? cw[i0 + tid] : 0.0;
+#pragma unroll
+                for (int d = 1; d < 64; d <<= 1) {
+                    const double u = __shfl_up(v, d);
+                    if (tid >= d) v += u;
                 }
+                if (i0 + tid < n) cw[i0 + tid] = c + v;
+                c += __shfl(v, 63);
+            }
         }
-        const double w = fw + cnt;
-        if (w == 0) {
-            fw = 0; fmean = 0; fm2 = 0;
-        } else {
-            const double w_safe = fmax_d(w, 2.2250738585072014e-308);
-            const double delta = pm_mean - fmean;
-            const double nm = fmean + delta * cnt / w_safe;
-            const double n2 = fm2 + pm_m2 + delta * delta * fw * cnt / w_safe;
-            fw = w; fmean = nm; fm2 = n2;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kStatsTile / kStatsT; k++) {
+            const int i = tid + kStatsT * k;
+            double term = 0.0;  // zeros past the tile: chain_sum's padding
+            if (i < n) {
+                const double before = i > 0 ? cw[i - 1] : cum_w0, w = cw[i] - before;
+                const double mean = cx[i] / fmax_d(cw[i], 1.0);
+                const double prev = i > 0 ? cx[i - 1] / fmax_d(before, 1.0) : mean_in;
+                term = (xv[k] - prev) * (xv[k] - mean) * w;
+                if ((i + 1) % ps == 0) {
+                    p.loc[(int64_t)r * p.cap_p + pt0 + i / ps] = (float)mean;
+                    pm_inv[i / ps] = 1.0 / fmax_d(fold_w0 + (cw[i] - cum_w0), 2.2250738585072014e-308);
+                }
+                if (i == n - 1) st_s[3] = mean;
+            }
+            sx[i] = term;
         }
+        __syncthreads();
+        if (tid == 0) {
+            st_s[2] = chain_sum(sx, sx, n, st_s[2]);
+            st_s[0] = cw[n - 1];
+        } else if (tid == 64) {
+            // welfordCombine (forecaster.zig:567-577), its mean: a division by the running count w per
+            // patch. a / w from y = 1 / w (rounded): q = a y, then q + (a - w q) y is the rounded
+            // quotient (Markstein's theorem); values past its range divide.
+            double fw = fold_w0, fmean = fo_s[1];
+#pragma unroll 4
+            for (int q = 0; q < np; q++) {
+                const double cnt = pm_cnt[q], w = fmax_d(fw + cnt, 2.2250738585072014e-308), y = pm_inv[q];
+                const double delta = pm_mean[q] - fmean, a = delta * cnt, q0 = a * y;
+                const double quo = __builtin_fma(__builtin_fma(-w, q0, a), y, q0);
+                fmean = fmean + (fabs(q0) > 1e-280 && fabs(q0) < 1e300 ? quo : a / w);
+                fw = fw + cnt;
+                pm_mean[q] = delta;
+            }
+            fo_s[1] = fmean;
+        }
+        __syncthreads();
+        for (int q = tid; q < np; q += kStatsT) {
+            const double cum_w = cw[q * ps + ps - 1], den = fmax_d(cum_w, 1.0), cnt = pm_cnt[q];
+            const double variance = sx[q * ps + ps - 1] / fmax_d(den - 1.0, 1.0);
+            p.scale[(int64_t)r * p.cap_p + pt0 + q] = (float)fmax_d(sqrt(variance), p.min_scale);
+            p.key_valid[(int64_t)r * p.cap_p + pt0 + q] = (uint8_t)(p.attend_missing ? pt0 + q >= first_s : cnt > 0);
+            // The fold's term of m2, delta^2 w_before cnt / w.
+            const double w = fold_w0 + (cum_w - cum_w0), delta = pm_mean[q];
+            pm_inv[q] = delta * delta * (w - cnt) * cnt / fmax_d(w, 2.2250738585072014e-308);
+        }
+        __syncthreads();
+        if (tid == 0) {
+            double fm2 = fo_s[2];
+#pragma unroll 8
+            for (int q = 0; q < np; q++) fm2 = fm2 + pm_m2[q] + pm_inv[q];
+            fo_s[2] = fm2;
+            fo_s[0] = fold_w0 + (cw[n - 1] - cum_w0);
+        }
+        __syncthreads();
     }
-    st[0] = cum_w; st[1] = cum_x; st[2] = m2; st[3] = prev_mean;
-    fo[0] = fw; fo[1] = fmean; fo[2] = fm2;
-    p.row_first[r] = first;
+    if (tid < 4) st[tid] = st_s[tid];
+    else if (tid < 7) fo[tid - 4] = fo_s[tid - 4];
+    else if (tid == 7) p.row_first[r] = first_s == 0x7fffffff ? -1 : first_s;
 }
 
 // predictBlock's patch features (model.zig:281-328) of patches [p0, l): values normalised by their
@@ -407,39 +525,61 @@ __global__ void ts_head_finish(const float* raw, const float* loc, const float* 
     for (int i = 0; i < q; i++) o[i] = ov[i];
 }
 
-// refineBlock's frames (src/timestral/forecaster.zig:602-652), one thread per row: fold the block's
-// medians (in the context's last-patch frame) patch by patch into the context's Welford state;
-// frames[r, j] = (loc_j, scale_j), patch 0 keeping (loc0, scale0).
-__global__ void ts_refine_frames(const float* qs, const float* loc, const float* scale, int cap_p, int l,
-                                 const double* fold, int rows, int h, int ps, int q, int median, double min_scale,
-                                 float* frames) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
+// refineBlock's frames (src/timestral/forecaster.zig:602-652): fold the block's medians (in the
+// context's last-patch frame) patch by patch into the context's Welford state; frames[r, j] =
+// (loc_j, scale_j), patch 0 keeping (loc0, scale0). One wave per row, a lane per step of the patch
+// (ps <= 256: four a lane at most): the medians' divisions and their maps into the frame are
+// spread over the lanes and the two sums of a patch are walked in the reference's order, by every
+// lane alike (one thread per row: 130 us a block of 32 patches; now 27 us).
+__global__ __launch_bounds__(64) void ts_refine_frames(const float* qs, const float* loc, const float* scale, int cap_p,
+                                                       int l, const double* fold, int h, int ps, int q, int median,
+                                                       double min_scale, float* frames) {
+    __shared__ double fs[256];
+    const int r = blockIdx.x, lane = threadIdx.x;
     const float loc0 = loc[(int64_t)r * cap_p + l - 1], scale0 = scale[(int64_t)r * cap_p + l - 1];
-    double w = fold[r * 3 + 0], mean = fold[r * 3 + 1], m2 = fold[r * 3 + 2];
+    double w = fold[(int64_t)r * 3 + 0], mean = fold[(int64_t)r * 3 + 1], m2 = fold[(int64_t)r * 3 + 2];
     const double clip = sqrt((double)3.40282347e38f) / 1e3, offset = mean;
     const float* block = qs + (int64_t)r * h * ps * q;
     float* fr = frames + (int64_t)r * h * 2;
+    auto frame_units = [&](int j, int k) {
+        return ((double)block[(int64_t)(j * ps + k) * q + median] - (double)loc0) / (double)scale0;
+    };
+    double sm[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) sm[e] = lane + 64 * e < ps ? frame_units(0, lane + 64 * e) : 0.0;
     for (int j = 0; j < h; j++) {
         const double variance = fmax_d(m2 / fmax_d(w - 1.0, 1.0), 0.0);
         const double sc = fmax_d(sqrt(variance), min_scale);
-        fr[2 * j] = (float)mean;
-        fr[2 * j + 1] = (float)sc;
-        // The block's medians of patch j mapped into this frame (computed twice: once for their
-        // mean, once for the squared deviations).
-        auto folded = [&](int k) {
-            const double sm = ((double)block[(j * ps + k) * q + median] - (double)loc0) / (double)scale0;
-            const double v = sm * sc + mean - offset;
-            return fmax_d(-clip, fmin(v, clip)) + offset;
-        };
-        double bsum = 0;
-        for (int k = 0; k < ps; k++) bsum += folded(k);
-        const double bmean = bsum / (double)ps;
-        double bm2 = 0;
-        for (int k = 0; k < ps; k++) {
-            const double f = folded(k);
-            bm2 += (f - bmean) * (f - bmean);
+        if (lane == 0) {
+            fr[2 * j] = j == 0 ? loc0 : (float)mean;
+            fr[2 * j + 1] = j == 0 ? scale0 : (float)sc;
         }
+        // The block's medians of patch j mapped into this frame.
+        double f[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const double v = sm[e] * sc + mean - offset;
+            f[e] = fmax_d(-clip, fmin(v, clip)) + offset;
+            if (lane + 64 * e < ps) fs[lane + 64 * e] = f[e];
+        }
+        if (j + 1 < h) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) sm[e] = lane + 64 * e < ps ? frame_units(j + 1, lane + 64 * e) : 0.0;
+        }
+        __syncthreads();
+        double bsum = 0;
+#pragma unroll 8
+        for (int k = 0; k < ps; k++) bsum += fs[k];
+        const double bmean = bsum / (double)ps;
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (lane + 64 * e < ps) fs[lane + 64 * e] = (f[e] - bmean) * (f[e] - bmean);
+        __syncthreads();
+        double bm2 = 0;
+#pragma unroll 8
+        for (int k = 0; k < ps; k++) bm2 += fs[k];
+        __syncthreads();
         // welfordCombine(state, (ps, bmean, bm2))
         const double bw = (double)ps, nw = w + bw;
         if (nw == 0) {
@@ -452,8 +592,6 @@ __global__ void ts_refine_frames(const float* qs, const float* loc, const float*
             w = nw; mean = nm; m2 = n2;
         }
     }
-    fr[0] = loc0;
-    fr[1] = scale0;
 }
 
 // refineBlock's rescale (forecaster.zig:653-659): (x - loc0) / scale0 * scale_j + loc_j, then
@@ -519,16 +657,22 @@ __global__ void ts_slide(const float* src, const uint8_t* src_mask, float* dst, 
 
 // forecastRaw's quantile cap (forecaster.zig:396-418) bounds of each row from its original context:
 // [min - a, max + a] over the observed values (0 when none), a = scale of the last patch x cap_k.
-__global__ void ts_cap_bounds(const float* ctx, const uint8_t* mask, int cap_t, int t, int ps, const float* scale,
-                              int cap_p, int rows, float cap_k, float* bounds) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= rows) return;
+// One wave per row (a thread per row: 228 us at 24 rows x 1504 steps; now 7 us).
+__global__ __launch_bounds__(64) void ts_cap_bounds(const float* ctx, const uint8_t* mask, int cap_t, int t, int ps,
+                                                    const float* scale, int cap_p, float cap_k, float* bounds) {
+    const int r = blockIdx.x, lane = threadIdx.x;
     float mx = -INFINITY, mn = INFINITY;
-    for (int j = 0; j < t; j++)
+    for (int j = lane; j < t; j += 64)
         if (mask[(int64_t)r * cap_t + j]) {
             mx = fmaxf(mx, ctx[(int64_t)r * cap_t + j]);
             mn = fminf(mn, ctx[(int64_t)r * cap_t + j]);
         }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        mx = fmaxf(mx, __shfl_xor(mx, d));
+        mn = fminf(mn, __shfl_xor(mn, d));
+    }
+    if (lane != 0) return;
     if (isinf(mx)) mx = 0.f;
     if (isinf(mn)) mn = 0.f;
     const float a = scale[(int64_t)r * cap_p + t / ps - 1] * cap_k;
@@ -571,7 +715,7 @@ unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per)
 }  // namespace
 
 hipError_t launch_ts_stats(const TsStatsParams& p, hipStream_t s) {
-    hipLaunchKernelGGL(ts_stats, dim3(blocks_for(p.rows, 64)), dim3(64), 0, s, p);
+    hipLaunchKernelGGL(ts_stats, dim3((unsigned)p.rows), dim3(kStatsT), 0, s, p);
     return hipGetLastError();
 }
 
@@ -624,8 +768,9 @@ hipError_t launch_ts_head_finish(const float* raw, const float* loc, const float
 hipError_t launch_ts_refine(float* qs, const float* loc, const float* scale, int cap_p, int l, const double* fold,
                             int rows, int h, int ps, int q, int median, double min_scale, float* frames,
                             hipStream_t s) {
-    hipLaunchKernelGGL(ts_refine_frames, dim3(blocks_for(rows, 64)), dim3(64), 0, s, qs, loc, scale, cap_p, l, fold, rows,
-                       h, ps, q, median, min_scale, frames);
+    if (ps > 256) return hipErrorInvalidValue;  // four steps a lane
+    hipLaunchKernelGGL(ts_refine_frames, dim3((unsigned)rows), dim3(64), 0, s, qs, loc, scale, cap_p, l, fold, h, ps, q,
+                       median, min_scale, frames);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(ts_refine_apply, dim3(blocks_for((int64_t)rows * h * ps, 128)), dim3(128), 0, s, qs, frames, rows,
@@ -656,8 +801,8 @@ hipError_t launch_ts_slide(const float* src, const uint8_t* src_mask, float* dst
 
 hipError_t launch_ts_cap_bounds(const float* ctx, const uint8_t* mask, int cap_t, int t, int ps, const float* scale,
                                 int cap_p, int rows, float cap_k, float* bounds, hipStream_t s) {
-    hipLaunchKernelGGL(ts_cap_bounds, dim3(blocks_for(rows, 64)), dim3(64), 0, s, ctx, mask, cap_t, t, ps, scale, cap_p,
-                       rows, cap_k, bounds);
+    hipLaunchKernelGGL(ts_cap_bounds, dim3((unsigned)rows), dim3(64), 0, s, ctx, mask, cap_t, t, ps, scale, cap_p, cap_k,
+                       bounds);
     return hipGetLastError();
 }
 
