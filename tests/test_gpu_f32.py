@@ -396,3 +396,26 @@ def test_repeatable_and_batch_independent(ta, gpu_ready):
     one = run_generic(ta, 1, np.ascontiguousarray(q[5:6]), np.ascontiguousarray(k[5:6]),
                       np.ascontiguousarray(v[5:6]), np.ascontiguousarray(kv[5:6]), 1, H, n, n, 0.125)
     assert np.array_equal(one[0], a[5])
+
+
+@pytest.mark.parametrize("mask", [0, 1, 4, 5])
+@pytest.mark.parametrize("n_q,n_k", [(7, 24), (8, 24), (24, 24), (32, 47), (33, 33), (64, 64), (65, 65), (66, 66),
+                                     (97, 97), (128, 144)])
+def test_short_rows_on_both_sides_of_the_kernel_choice(ta, gpu_ready, mask, n_q, n_k):
+    """Rows of at most 144 keys run on the resident f32 kernel or the bf16x3 one by row count and
+    length: 258 rows (more than the CUs of the GPU, three of them checked) and 2, on both sides of
+    each length at which the choice changes, against float64."""
+    H = 6
+    for B in (43, 1):
+        q, k, v, kv = _inputs(n_q + 10 * n_k + B, B, H, n_q, n_k)
+        extra = dict(q_pos0=n_k - n_q) if mask >= 2 else {}
+        if mask == 5:
+            extra.update(ctx_keys=n_k - n_q, chain_start=n_k - n_q)
+        heads = H if B > 1 else 2
+        got = run_generic(ta, mask, *(np.ascontiguousarray(a[:, :, :heads * 64]) for a in (q, k, v)), kv, B, heads,
+                          n_q, n_k, 0.125, **extra)
+        for b, h in ((0, 0), (B // 2, 1), (B - 1, heads - 1)):
+            sel = slice(h * 64, h * 64 + 64)
+            allowed = _ref.allowed_matrix(mask, n_q, n_k, kv[b], **extra)
+            want = _ref.naive_attend(q[b, :, sel], k[b, :, sel], v[b, :, sel], allowed, 0.125)
+            assert _ref.scaled_err(got[b, :, sel], want) <= TOL, (B, b, h)
