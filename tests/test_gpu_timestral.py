@@ -414,3 +414,32 @@ def test_timestral_rows_longer_than_a_tile(ta, orc, orc16, gpu_ready, length, ps
     w8, w16 = (_oracle(o_, m, x, obs, b, v, horizon, 0, 2) for o_ in (orc, orc16))
     assert np.isfinite(got).all()
     _ref.assert_within_reference_bar(got, w8, w16, _ref.timestral_forecast_f64(m, x, obs, b, v, horizon, per_shot=2))
+
+
+@pytest.mark.parametrize("b,v,hid,gated,kv_cache,use_asinh", [(32, 1, 96, True, True, True), (17, 2, 160, True, True, False),
+                                                             (32, 1, 96, False, True, True),
+                                                             (13, 2, 128, True, False, True)])
+def test_timestral_weights_split_once_per_call(ta, orc, orc16, gpu_ready, b, v, hid, gated, kv_cache, use_asinh):
+    """Forecasts of several decode blocks with at least 2048 tokens in all: the layers' weights are split
+    once per call, the norms, gates and MLP activations written split for the products of the blocks
+    of at least 768 tokens (ragged row blocks, hidden widths of 3 to 5 chunks, with and without
+    gates), the shorter blocks splitting inside their products. Against both oracle builds and
+    float64; in bf16 against the f32 forecast."""
+    length, horizon, per_shot = 470, 80, 3
+    rng = np.random.default_rng(b + hid)
+    m = _ref.timestral_model(rng, d=128, nh=2, hid=hid, schedule=("time_variate", "time"), use_asinh=use_asinh,
+                             gated=gated)
+    t = np.arange(length)
+    x = (20 + 6 * np.sin(2 * np.pi * t / 24) + 0.02 * t + rng.standard_normal((b * v, length))).astype(np.float32)
+    obs = rng.random((b * v, length)) >= 0.1
+    x[~obs] = 0
+    rows = 2 * b * v  # blocks of 3 and 2 patches after 30 of context
+    assert rows * (30 + 3) >= 768 and rows * (30 + 3 + (3 if kv_cache else 33) + 2) >= 2048
+    got = _gpu(ta, m, x, obs, b, v, horizon, per_shot=per_shot, kv_cache=kv_cache)
+    w8, w16 = (_oracle(o_, m, x, obs, b, v, horizon, 0, per_shot) for o_ in (orc, orc16))
+    exact = _ref.timestral_forecast_f64(m, x, obs, b, v, horizon, per_shot=per_shot)
+    assert np.isfinite(got).all()
+    _ref.assert_within_reference_bar(got, w8, w16, exact)
+    if not use_asinh:
+        half = _gpu(ta, m, x, obs, b, v, horizon, per_shot=per_shot, kv_cache=kv_cache, attn_bf16=True)
+        assert _ref.scaled_err(half, w16) < 1e-2

@@ -96,6 +96,10 @@ struct ProjParams {
     // result written split (one f32 output, width a multiple of 32, no RoPE) instead of into y0.
     const void* x_pre;
     void* y_planes;
+    // Optional: the weights already split (launch_weight_planes of w0; of w0 .. w3 one after the other with
+    // several outputs, each a multiple of 16 rows; they are then not read), for a caller that uses
+    // them in several products. The product runs on pre-split operands whatever its size.
+    const void* w_pre;
     // Optional row norm of the finished product (one f32 output): norm_out = rmsNorm(y0, norm_scale,
     // norm_eps), the same arithmetic as launch_rms_norm; may be y0 itself.
     const float* norm_scale;
@@ -153,6 +157,13 @@ bool proj_planes_ready(int64_t tokens, int64_t d_in, int64_t n_cols);
 // (dim a multiple of 32).
 hipError_t launch_rms_norm_planes(const float* x, int64_t x_tok, void* planes, const float* scale, int rows, int dim,
                                   float eps, hipStream_t stream);
+// x / (1 + exp(-g)) over rows x cols, written split for a product (x_pre); x and g at row stride tok.
+hipError_t launch_mul_sigmoid_planes(const float* x, const float* g, int64_t tok, void* planes, int rows, int cols,
+                                     hipStream_t stream);
+// gate * silu(up) of h = [gate | up] rows (2 hid wide), written split for a product (x_pre).
+hipError_t launch_mul_silu_planes(const float* h, void* planes, int rows, int hid, hipStream_t stream);
+// A (rows x cols) weight split for w_pre.
+hipError_t launch_weight_planes(const float* w, int64_t w_ld, int rows, int cols, void* planes, hipStream_t stream);
 class PlaneWorkspace {
 public:
     PlaneWorkspace(void* buf, size_t bytes);

@@ -534,27 +534,28 @@ __global__ __launch_bounds__(256) void split_planes(SplitSrc s, uint8_t* __restr
     *reinterpret_cast<u32x4*>(out + 2 * kPlaneChunk) = u32x4{l0[0], l0[1], l1[0], l1[1]};
 }
 
-// rmsNorm of 16 rows per workgroup into the pre-split layout: each wave reduces four rows with the
-// lane mapping of rms_norm_rows (so the norms are the same bits), then the workgroup writes the
-// rows' chunks, 1 KB per wave at a time.
-__global__ __launch_bounds__(256) void rms_norm_planes(const float* __restrict__ x, int64_t x_tok,
-                                                       uint8_t* __restrict__ dst, const float* __restrict__ scale,
-                                                       int rows, int dim, float eps) {
+// rmsNorm of 16 rows per workgroup into the pre-split layout: each wave reduces one row with the lane
+// mapping of rms_norm_rows (so the norms are the same bits), then the workgroup writes the rows'
+// chunks, 1 KB per wave at a time. Bound by HBM when there are rows for every CU (36928 rows of 768:
+// 57.5 us for 283 MB), by a wave's chain of loads with fewer. Four waves of four rows each took 66.3
+// there and 14.5 at 3024 rows of 1024, where sixteen take 10.1.
+constexpr int kNormWaves = 16;
+__global__ __launch_bounds__(64 * kNormWaves) void rms_norm_planes(const float* __restrict__ x, int64_t x_tok,
+                                                                   uint8_t* __restrict__ dst,
+                                                                   const float* __restrict__ scale, int rows, int dim,
+                                                                   float eps) {
     __shared__ float inv_s[16];
     const int rb = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int r = 4 * wave + i, row = rb * 16 + r;
-        if (row >= rows) continue;  // wave-uniform
-        const float* xr = x + (int64_t)row * x_tok;
+    if (rb * 16 + wave < rows) {  // wave-uniform
+        const float* xr = x + (int64_t)(rb * 16 + wave) * x_tok;
         float ss = 0.f;
         for (int c = 4 * lane; c < dim; c += 256) ss = sumsq4(ss, ld4(xr + c));
         const float inv = rms_inv(ss, dim, eps);
-        if (lane == 0) inv_s[r] = inv;
+        if (lane == 0) inv_s[wave] = inv;
     }
     __syncthreads();
     const int kc = dim / X3_BK, r = lane & 15, row = rb * 16 + r;
-    for (int k = wave; k < kc; k += 4) {
+    for (int k = wave; k < kc; k += kNormWaves) {
         const int c0 = k * X3_BK + 8 * (lane >> 4);
         f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
         if (row < rows) {
@@ -570,6 +571,42 @@ __global__ __launch_bounds__(256) void rms_norm_planes(const float* __restrict__
         *reinterpret_cast<u32x4*>(out + kPlaneChunk) = u32x4{m0[0], m0[1], m1[0], m1[1]};
         *reinterpret_cast<u32x4*>(out + 2 * kPlaneChunk) = u32x4{l0[0], l0[1], l1[0], l1[1]};
     }
+}
+
+// The elementwise steps ahead of a product, written straight into the pre-split layout (one pass where
+// the step's own f32 result would be written, read back and split): nn.mulSigmoid of the time
+// attention's output, x / (1 + exp(-g)), and MlpAct.run, gate * (up / (1 + exp(-up))) with gate = x
+// and up = g (src/core/nn.zig:410-433). Same arithmetic as the f32 kernels (ts_mul_sigmoid,
+// ts_mul_silu), so the same bits. Bound by HBM / L2 traffic. At 3024 rows, gate step of 1024
+// columns: 7.4 us + 6.9 us of split before, 9.5 us now; SiLU step of 2816: 16.2 + 14.3, 20.6 us now.
+enum { kActGate = 0, kActMlp = 1 };
+template <int ACT>
+__global__ __launch_bounds__(256) void act_planes(const float* __restrict__ x, const float* __restrict__ g, int64_t ld,
+                                                  uint8_t* __restrict__ dst, int rows, int kc) {
+#pragma clang fp contract(off)
+    const int64_t c = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // chunk (rb, k)
+    const int lane = threadIdx.x & 63;
+    if (c >= (int64_t)((rows + 15) / 16) * kc) return;
+    const int rb = (int)(c / kc), k = (int)(c - (int64_t)rb * kc);
+    const int row = rb * 16 + (lane & 15);
+    f32x4 v[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    if (row < rows) {
+        const int64_t at = row * ld + k * X3_BK + 8 * (lane >> 4);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const f32x4 xv = ld4(x + at + 4 * h), gv = ld4(g + at + 4 * h);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                v[h][i] = ACT == kActGate ? xv[i] / (1.f + expf(-gv[i])) : xv[i] * (gv[i] / (1.f + expf(-gv[i])));
+        }
+    }
+    u32x2 h0, m0, l0, h1, m1, l1;
+    split3(v[0], h0, m0, l0);
+    split3(v[1], h1, m1, l1);
+    uint8_t* const out = dst + c * 3 * kPlaneChunk + 16 * lane;
+    *reinterpret_cast<u32x4*>(out) = u32x4{h0[0], h0[1], h1[0], h1[1]};
+    *reinterpret_cast<u32x4*>(out + kPlaneChunk) = u32x4{m0[0], m0[1], m1[0], m1[1]};
+    *reinterpret_cast<u32x4*>(out + 2 * kPlaneChunk) = u32x4{l0[0], l0[1], l1[0], l1[1]};
 }
 
 template <int OUT, bool BIG>
@@ -967,10 +1004,15 @@ size_t plane_operand_bytes(int64_t rows, int64_t cols) {
     if (rows <= 0 || cols <= 0 || cols % X3_BK) return 0;
     return (size_t)((rows + 15) / 16) * (size_t)(cols / X3_BK) * 3 * kPlaneChunk;
 }
-// Products of at least 2^30 multiply-adds run on pre-split operands when a workspace is lent: the
-// split launches cost more than they save on smaller ones.
+// Products that run on pre-split operands when a workspace is lent: at least 2^30 multiply-adds over
+// at least 2048 rows, or 5 2^30 over fewer. Splitting the weights costs the same at any row count
+// and saves each row tile its own split, so it pays by rows (whole calls in us, pre-split / split
+// inside the product: Chronos-2 layers of 484 rows 500 / 457, 1205 rows 675 / 634, 1928 rows 886 / 867,
+// 4820 rows 1513 / 1707; Timestral q/k/v/gate, 4096 columns: 333 rows 43 / 39, 999 rows 62 / 57, 1332
+// rows 87 / 93).
 static bool planes_pay(int64_t tokens, int64_t d_in, int64_t n_cols) {
-    return d_in % X3_BK == 0 && tokens * n_cols * d_in >= ((int64_t)1 << 30);
+    const int64_t macs = tokens * n_cols * d_in, unit = (int64_t)1 << 30;
+    return d_in % X3_BK == 0 && macs >= unit && (tokens >= 2048 || macs >= 5 * unit);
 }
 bool proj_planes_ready(int64_t tokens, int64_t d_in, int64_t n_cols) {
     return t_plane_ws != nullptr && planes_pay(tokens, d_in, n_cols) &&
@@ -980,8 +1022,39 @@ hipError_t launch_rms_norm_planes(const float* x, int64_t x_tok, void* planes, c
                                   float eps, hipStream_t stream) {
     if (rows <= 0) return hipSuccess;
     if (dim <= 0 || dim % X3_BK) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(rms_norm_planes, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, stream, x, x_tok,
+    hipLaunchKernelGGL(rms_norm_planes, dim3((unsigned)((rows + 15) / 16)), dim3(64 * kNormWaves), 0, stream, x, x_tok,
                        static_cast<uint8_t*>(planes), scale, rows, dim, eps);
+    return hipGetLastError();
+}
+
+namespace {
+template <int ACT>
+hipError_t launch_act_planes(const float* x, const float* g, int64_t ld, void* planes, int rows, int cols,
+                             hipStream_t stream) {
+    if (rows <= 0 || cols <= 0) return hipSuccess;
+    if (cols % X3_BK) return hipErrorInvalidValue;
+    const int kc = cols / X3_BK;
+    const int64_t chunks = (int64_t)((rows + 15) / 16) * kc;
+    hipLaunchKernelGGL((act_planes<ACT>), dim3((unsigned)((chunks + 3) / 4)), dim3(256), 0, stream, x, g, ld,
+                       static_cast<uint8_t*>(planes), rows, kc);
+    return hipGetLastError();
+}
+}  // namespace
+hipError_t launch_mul_sigmoid_planes(const float* x, const float* g, int64_t tok, void* planes, int rows, int cols,
+                                     hipStream_t stream) {
+    return launch_act_planes<kActGate>(x, g, tok, planes, rows, cols, stream);
+}
+hipError_t launch_mul_silu_planes(const float* h, void* planes, int rows, int hid, hipStream_t stream) {
+    return launch_act_planes<kActMlp>(h, h + hid, 2 * (int64_t)hid, planes, rows, hid, stream);
+}
+hipError_t launch_weight_planes(const float* w, int64_t w_ld, int rows, int cols, void* planes, hipStream_t stream) {
+    if (rows <= 0 || cols <= 0) return hipSuccess;
+    if (cols % X3_BK) return hipErrorInvalidValue;
+    const int kc = cols / X3_BK;
+    const SplitSrc src = {{w, w, w, w}, w_ld, rows, rows, kc};
+    const int64_t chunks = (int64_t)((rows + 15) / 16) * kc;
+    hipLaunchKernelGGL(split_planes, dim3((unsigned)((chunks + 3) / 4)), dim3(256), 0, stream, src,
+                       static_cast<uint8_t*>(planes));
     return hipGetLastError();
 }
 
@@ -1092,7 +1165,7 @@ static int proj_chunk(int units) {
 // Products the 16-token kernel takes (proj_skinny).
 static bool skinny(const ProjParams& p) {
     return p.tokens <= kSkinnyTokens && p.d_in <= kSkinnyMaxIn && p.rope_cos == nullptr && p.out_dtype == 0 &&
-           p.x_pre == nullptr && p.y_planes == nullptr;
+           p.x_pre == nullptr && p.y_planes == nullptr && p.w_pre == nullptr;
 }
 
 bool proj_fuses_input_norm(int64_t tokens, int64_t d_in) {
@@ -1107,7 +1180,7 @@ size_t proj_split_bytes(ProjParams& p) {
     p.splits = 1;
     p.split_steps = steps;
     p.partial = nullptr;
-    if (p.x_pre != nullptr || p.y_planes != nullptr) return 0;  // pre-split operands: never split
+    if (p.x_pre != nullptr || p.y_planes != nullptr || p.w_pre != nullptr) return 0;  // pre-split operands: never split
     // f32 outputs, no RoPE; several outputs only without an epilogue; at most half a launch of
     // tiles (four workgroups per CU), and at least 16 steps to share out.
     if (!((p.n_out == 1 || p.epi == kEpiNone) && p.rope_cos == nullptr && p.out_dtype == 0 && blocks < 512 &&
@@ -1158,31 +1231,37 @@ hipError_t launch_proj(const ProjParams& p0, hipStream_t stream) {
         return e;
     }
     // Pre-split operands when the entry point lent a large enough PlaneWorkspace: the weights split
-    // into it, and x too unless its producer split it (x_pre). x_pre / y_planes need that path.
+    // into it (unless the caller has them split already, w_pre), and x too unless its producer split it
+    // (x_pre). x_pre / y_planes / w_pre need that path.
     p.xp = p.wp = nullptr;
     const int64_t n_cols = (int64_t)p.width * p.n_out;
-    const bool fused = p.x_pre != nullptr || p.y_planes != nullptr;
-    if (fused && (!proj_planes_ready(p.tokens, p.d_in, n_cols) ||
-                  (p.y_planes != nullptr && (p.n_out != 1 || p.width % X3_BK || p.out_dtype != 0 || p.rope_cos != nullptr))))
+    const bool ready = p.w_pre != nullptr ? p.d_in % X3_BK == 0 : proj_planes_ready(p.tokens, p.d_in, n_cols);
+    if (((p.x_pre != nullptr || p.y_planes != nullptr || p.w_pre != nullptr) && !ready) ||
+        (p.y_planes != nullptr && (p.n_out != 1 || p.width % X3_BK || p.out_dtype != 0 || p.rope_cos != nullptr)))
         return hipErrorInvalidValue;
-    if (t_plane_ws != nullptr && planes_pay(p.tokens, p.d_in, n_cols)) {
+    if (p.w_pre != nullptr || (t_plane_ws != nullptr && planes_pay(p.tokens, p.d_in, n_cols))) {
         const size_t xb = p.x_pre != nullptr ? 0 : plane_operand_bytes(p.tokens, p.d_in);
-        if (xb + plane_operand_bytes(n_cols, p.d_in) <= t_plane_bytes) {
+        const size_t wb = p.w_pre != nullptr ? 0 : plane_operand_bytes(n_cols, p.d_in);
+        if (xb + wb <= (t_plane_ws != nullptr ? t_plane_bytes : 0)) {
             const int kc = p.d_in / X3_BK;
             uint8_t* const xp = static_cast<uint8_t*>(t_plane_ws);
             uint8_t* const wp = xp + xb;
-            SplitSrc sw = {{p.w0, p.w1 ? p.w1 : p.w0, p.w2 ? p.w2 : p.w0, p.w3 ? p.w3 : p.w0}, p.w_ld, p.width,
-                           (int32_t)n_cols, kc};
-            if (p.x_pre == nullptr) {
+            if (xb > 0) {
                 SplitSrc sx = {{p.x, p.x, p.x, p.x}, p.x_tok, p.tokens, p.tokens, kc};
                 const int64_t cx = (int64_t)((p.tokens + 15) / 16) * kc;
                 hipLaunchKernelGGL(split_planes, dim3((unsigned)((cx + 3) / 4)), dim3(256), 0, stream, sx, xp);
             }
-            const int64_t cw = (n_cols + 15) / 16 * kc;
-            hipLaunchKernelGGL(split_planes, dim3((unsigned)((cw + 3) / 4)), dim3(256), 0, stream, sw, wp);
+            if (wb > 0) {
+                SplitSrc sw = {{p.w0, p.w1 ? p.w1 : p.w0, p.w2 ? p.w2 : p.w0, p.w3 ? p.w3 : p.w0}, p.w_ld, p.width,
+                               (int32_t)n_cols, kc};
+                const int64_t cw = (n_cols + 15) / 16 * kc;
+                hipLaunchKernelGGL(split_planes, dim3((unsigned)((cw + 3) / 4)), dim3(256), 0, stream, sw, wp);
+            }
             if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
             p.xp = p.x_pre != nullptr ? p.x_pre : xp;
-            p.wp = wp;
+            p.wp = p.w_pre != nullptr ? p.w_pre : wp;
+        } else if (p.x_pre != nullptr || p.w_pre != nullptr) {
+            return hipErrorInvalidValue;
         }
     }
     // Small products (a few token tiles: the decoder's 16 rows, short encoders) leave most CUs idle

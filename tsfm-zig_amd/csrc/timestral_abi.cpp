@@ -40,13 +40,22 @@ namespace {
 
 constexpr int kActSilu = 1;  // tsfm_resblock.act
 
+// The kept weight planes of a call: from this many tokens over all its blocks, up to this many bytes;
+// a block of fewer than kWeightPlanesBlock tokens splits inside its products instead, where the
+// reduction is shared out over more workgroups.
+constexpr int64_t kWeightPlanesTokens = 2048;
+constexpr int64_t kWeightPlanesBlock = 768;
+constexpr size_t kWeightPlanesMax = (size_t)4 << 30;
+
 // One nn.linear (y = x w^T + bias) with an epilogue, over `rows` packed rows.
 hipError_t linear(const float* x, int64_t x_tok, const float* w, int out, int in, const float* bias, float* y,
-                  int64_t y_tok, int rows, int epi, const float* resid, hipStream_t s) {
+                  int64_t y_tok, int rows, int epi, const float* resid, hipStream_t s, const void* x_pre = nullptr,
+                  const void* w_pre = nullptr) {
     tsfm::ProjParams p{};
     p.x = x; p.x_tok = x_tok; p.w0 = w; p.w_ld = in; p.alpha = 1.f; p.epi = epi; p.bias = bias;
     p.resid = resid; p.resid_tok = y_tok;
     p.y0 = y; p.y0_tok = y_tok;
+    p.x_pre = x_pre; p.w_pre = w_pre;
     p.tokens = rows; p.seq = rows; p.d_in = in; p.width = out; p.n_out = 1; p.out_dtype = TSFM_DTYPE_F32;
     return tsfm::launch_proj(p, s);
 }
@@ -199,6 +208,20 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
     const int cap_t = t_first + total_patches * ps, cap_p = cap_t / ps;
     const int cap_tok = cap_p + per_shot + (cov ? per_shot : 0), sl_max = cap_tok;  // cov: window + decoder
     const int hpad = total_patches * ps;
+    const bool cached = a->kv_cache != 0 && a->n_known == 0;
+    // Tokens of all decode blocks together, as the loop below runs them.
+    auto total_tokens = [&]() {
+        int64_t n = 0;
+        for (int left = total_patches, t = t_first, p0 = 0; left > 0;) {
+            const int h = std::min(per_shot, left), l = t / ps;
+            n += (int64_t)rows * ((cov ? l + h : l) - p0 + h);
+            left -= h;
+            const bool drop = t + h * ps > max_context;
+            p0 = drop || !cached ? 0 : l;
+            t = drop ? std::max(ps, max_context / ps * ps) : t + h * ps;
+        }
+        return n;
+    };
     if ((int64_t)rows * cap_tok * 3 * d > 0x7fffffffLL * 4) return fail(TSFM_E_UNSUPPORTED, "too large");
     hipStream_t s = static_cast<hipStream_t>(a->stream);
 
@@ -226,6 +249,22 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
     const size_t at_part = plan.take(tsfm::kSplitWorkspaceBytes);
     const size_t planes_n = tsfm::proj_plane_bytes((int64_t)rows * sl_max, std::max(d, hid), std::max(3 * d, 2 * hid));
     const size_t at_planes = plan.take(planes_n);
+    // Pre-split operands (32-wide widths). at_xpl: the norms', gates' and MLP activations' results as the
+    // next product reads them. With several decode blocks, the layers' weights split once for the call (at_wpl)
+    // instead of once per block and product, when the blocks together are long enough to repay it and
+    // the copy (1.5x the weights) stays within kWeightPlanesMax.
+    const bool splits = d % 32 == 0 && hid % 32 == 0;
+    const int64_t call_tokens = total_tokens();
+    const size_t at_xpl = plan.take(splits ? tsfm::plane_operand_bytes((int64_t)rows * sl_max, std::max(d, hid)) : 0);
+    size_t wpl_n = 0;
+    for (int li = 0; li < M.n_layers; li++) {
+        for (int ai = 0; ai < M.layers[li].n_attn; ai++)
+            wpl_n += tsfm::plane_operand_bytes((M.layers[li].attn[ai].gate ? 5 : 4) * (int64_t)d, d);
+        wpl_n += tsfm::plane_operand_bytes(2 * (int64_t)hid, d) + tsfm::plane_operand_bytes(d, hid);
+    }
+    const bool keep_weights = splits && total_patches > per_shot && call_tokens >= kWeightPlanesTokens &&
+                              wpl_n <= kWeightPlanesMax;
+    const size_t at_wpl = plan.take(keep_weights ? wpl_n : 0);
     const size_t at_kf = plan.take((size_t)rows * hpad * 4 + 4), at_kfm = plan.take((size_t)rows * hpad + 1);
     const size_t at_noasinh = plan.take((size_t)rows);
     char* buf = nullptr;
@@ -275,11 +314,30 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
         cp.ctx = ctx[0]; cp.mask = mask[0]; cp.kf = F(at_kf); cp.kfm = U8(at_kfm); cp.nonneg = U8(at_nonneg);
         hipError_t e2 = tsfm::launch_ts_context(cp, s);
         if (e2 != hipSuccess) return e2;
+        // Per layer: each attention's q/k/v (and gate) weights, its out weight, then w12 and w3.
+        if (keep_weights) {
+            char* at = buf + at_wpl;
+            auto split = [&](const float* w, int64_t n, int64_t k) {
+                if (e2 != hipSuccess) return;
+                e2 = tsfm::launch_weight_planes(w, k, (int)n, (int)k, at, s);
+                at += tsfm::plane_operand_bytes(n, k);
+            };
+            for (int li = 0; li < M.n_layers; li++) {
+                const tsfm_timestral_layer& ly = M.layers[li];
+                for (int ai = 0; ai < ly.n_attn; ai++) {
+                    split(ly.attn[ai].qkv, 3 * (int64_t)d, d);
+                    if (ly.attn[ai].gate) split(ly.attn[ai].gate, d, d);
+                    split(ly.attn[ai].out, d, d);
+                }
+                split(ly.w12, 2 * (int64_t)hid, d);
+                split(ly.w3, d, hid);
+            }
+            if (e2 != hipSuccess) return e2;
+        }
         // Known-future rows attend over the whole window and take whole-window statistics: every
         // token changes when the window grows. Past-only rows are causal like the targets; their
         // blank future patches (read by no context token or decoder query) leave the carried
         // statistics unchanged (zero weight) and are recomputed as context in the next block.
-        const bool cache = a->kv_cache != 0 && a->n_known == 0;
         const int known_from = V + a->n_past;  // first known-future row of a series
         int t = t_first, remaining = total_patches, done = 0;
         int stats_from = 0;  // first step of the window whose statistics are not computed yet
@@ -326,15 +384,36 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
             // 3. the layers (runTransformer, model.zig:465-481)
             const int toks = rows * sl;
             int ti = 0;
+            // Which products of this block read their operands pre-split, and with kept weights.
+            const bool kept = keep_weights && toks >= kWeightPlanesBlock;
+            void* const XP = buf + at_xpl;
+            const char* wp = buf + at_wpl;
+            auto weights = [&](int64_t n, int64_t k) -> const void* {
+                const char* at = wp;
+                wp += tsfm::plane_operand_bytes(n, k);
+                return kept ? at : nullptr;
+            };
+            auto pre = [&](int64_t k, int64_t n) { return splits && (kept || tsfm::proj_planes_ready(toks, k, n)); };
             for (int li = 0; li < M.n_layers; li++) {
                 const tsfm_timestral_layer& ly = M.layers[li];
                 for (int ai = 0; ai < ly.n_attn; ai++) {
                     const tsfm_timestral_attn& at = ly.attn[ai];
-                    if ((e2 = tsfm::launch_rms_norm(X, d, XN, d, at.norm, toks, d, eps, s)) != hipSuccess) return e2;
+                    // The q/k/v (and gate) weights are one (4 d, d) operand of one product, or with bf16
+                    // q/k/v two products, whose parts lie in turn.
+                    const int n_out = at.gate && !(at.is_time && half) ? 4 : 3;
+                    const void* const wq = weights(3 * (int64_t)d, d);
+                    const void* const wg = at.gate ? weights(d, d) : nullptr;
+                    const void* const wo = weights(d, d);
+                    const bool pn = pre(d, n_out * (int64_t)d) && (n_out == 4 || !at.gate || pre(d, d));
+                    if ((e2 = pn ? tsfm::launch_rms_norm_planes(X, d, XP, at.norm, toks, d, eps, s)
+                                 : tsfm::launch_rms_norm(X, d, XN, d, at.norm, toks, d, eps, s)) != hipSuccess)
+                        return e2;
+                    bool po = false;  // the gated attention output is in XP, split
                     tsfm::ProjParams pp{};
+                    pp.x_pre = pn ? XP : nullptr; pp.w_pre = wq;
                     pp.x = XN; pp.x_tok = d; pp.w_ld = d; pp.alpha = 1.f; pp.epi = tsfm::kEpiNone;
                     pp.w0 = at.qkv; pp.w1 = at.qkv + (int64_t)d * d; pp.w2 = at.qkv + 2 * (int64_t)d * d; pp.w3 = at.gate;
-                    pp.tokens = toks; pp.seq = sl; pp.d_in = d; pp.width = d; pp.n_out = at.gate ? 4 : 3;
+                    pp.tokens = toks; pp.seq = sl; pp.d_in = d; pp.width = d; pp.n_out = n_out;
                     pp.out_dtype = TSFM_DTYPE_F32;
                     pp.y3 = G; pp.y3_tok = d;
                     if (at.is_time) {
@@ -347,7 +426,7 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
                         pp.y0 = el((int64_t)p0 * 3 * d); pp.y1 = el((int64_t)p0 * 3 * d + d);
                         pp.y2 = el((int64_t)p0 * 3 * d + 2 * d);
                         if (half) {  // q/k/v rounded to bf16; the gate stays f32 (its own product)
-                            pp.out_dtype = TSFM_DTYPE_BF16; pp.n_out = 3; pp.w3 = nullptr; pp.y3 = nullptr;
+                            pp.out_dtype = TSFM_DTYPE_BF16; pp.w3 = nullptr; pp.y3 = nullptr;
                         }
                         pp.y0_tok = pp.y1_tok = pp.y2_tok = 3 * d;
                         pp.y0_batch = pp.y1_batch = pp.y2_batch = tb;
@@ -355,8 +434,8 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
                         pp.rope_table_stride = (int64_t)cap_tok * 32; pp.rope_rows_per_table = vall; pp.rope_row0 = 0;
                         if ((e2 = tsfm::launch_proj(pp, s)) != hipSuccess) return e2;
                         if (half && at.gate &&
-                            (e2 = linear(XN, d, at.gate, d, d, nullptr, G, d, toks, tsfm::kEpiNone, nullptr, s)) !=
-                                hipSuccess)
+                            (e2 = linear(XN, d, at.gate, d, d, nullptr, G, d, toks, tsfm::kEpiNone, nullptr, s,
+                                         pn ? XP : nullptr, wg)) != hipSuccess)
                             return e2;
                         auto attend = [&](const tsfm::Params& q, int msk) {
                             return half ? tsfm::launch_attn_half(q, true, msk, tsfm::BIAS_NONE, false, s)
@@ -399,8 +478,11 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
                             if ((e2 = tsfm::launch_ts_from_bf16(OH, at.gate ? G : nullptr, OA, (int64_t)toks * d, s)) !=
                                 hipSuccess)
                                 return e2;
-                        } else if (at.gate && (e2 = tsfm::launch_ts_mul_sigmoid(OA, G, (int64_t)toks * d, s)) != hipSuccess) {
-                            return e2;
+                        } else if (at.gate) {
+                            po = pre(d, d);
+                            if ((e2 = po ? tsfm::launch_mul_sigmoid_planes(OA, G, d, XP, toks, d, s)
+                                         : tsfm::launch_ts_mul_sigmoid(OA, G, (int64_t)toks * d, s)) != hipSuccess)
+                                return e2;
                         }
                     } else {
                         // variateAttention (:525-544): the block's token slots only, gate fused.
@@ -417,14 +499,21 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
                         vp.scale = sm_scale;
                         if ((e2 = tsfm::launch_variate(vp, s)) != hipSuccess) return e2;
                     }
-                    if ((e2 = linear(OA, d, at.out, d, d, nullptr, X, d, toks, tsfm::kEpiResidual, X, s)) != hipSuccess)
+                    if ((e2 = linear(OA, d, at.out, d, d, nullptr, X, d, toks, tsfm::kEpiResidual, X, s,
+                                     po ? XP : nullptr, wo)) != hipSuccess)
                         return e2;
                 }
-                if ((e2 = tsfm::launch_rms_norm(X, d, XN, d, ly.mlp_norm, toks, d, eps, s)) != hipSuccess ||
-                    (e2 = linear(XN, d, ly.w12, 2 * hid, d, nullptr, H, 2 * hid, toks, tsfm::kEpiNone, nullptr, s)) !=
-                        hipSuccess ||
-                    (e2 = tsfm::launch_ts_mul_silu(H, A, toks, hid, s)) != hipSuccess ||
-                    (e2 = linear(A, hid, ly.w3, d, hid, nullptr, X, d, toks, tsfm::kEpiResidual, X, s)) != hipSuccess)
+                const void* const w12 = weights(2 * (int64_t)hid, d);
+                const void* const w3 = weights(d, hid);
+                const bool pn = pre(d, 2 * (int64_t)hid), pa = pre(hid, d);
+                if ((e2 = pn ? tsfm::launch_rms_norm_planes(X, d, XP, ly.mlp_norm, toks, d, eps, s)
+                             : tsfm::launch_rms_norm(X, d, XN, d, ly.mlp_norm, toks, d, eps, s)) != hipSuccess ||
+                    (e2 = linear(XN, d, ly.w12, 2 * hid, d, nullptr, H, 2 * hid, toks, tsfm::kEpiNone, nullptr, s,
+                                 pn ? XP : nullptr, w12)) != hipSuccess ||
+                    (e2 = pa ? tsfm::launch_mul_silu_planes(H, XP, toks, hid, s)
+                             : tsfm::launch_ts_mul_silu(H, A, toks, hid, s)) != hipSuccess ||
+                    (e2 = linear(A, hid, ly.w3, d, hid, nullptr, X, d, toks, tsfm::kEpiResidual, X, s,
+                                 pa ? XP : nullptr, w3)) != hipSuccess)
                     return e2;
             }
             // 4. the head on the decoder tokens, the monotone quantiles, refineBlock
@@ -458,7 +547,7 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
                 t = keep_t;
                 stats_from = 0;
                 p0 = 0;
-            } else if (cache) {
+            } else if (cached) {
                 stats_from = t;
                 p0 = l;
                 t = nt;
