@@ -535,3 +535,26 @@ def test_categorical_encoding_errors(ta, over, msg):
     a = ta.CategoricalArgs(**kw)
     assert ta.load().tsfm_timestral_encode_categorical(ta.ctypes.byref(a)) == ta.E_INVALID
     assert msg in ta.last_error()
+
+
+def test_make_args_fills_every_field():
+    """The packed argument block equals one filled field by field, values past their field included
+    (the conversion ctypes itself makes)."""
+    import numpy as np
+    import tsfm_attn as ta
+
+    q, kv = np.zeros(64, np.float32), np.zeros(4, np.uint8)
+    ints = dict(batch=2, heads=3, n_q=5, n_k=7, q_tok=64, q_batch=1 << 40, k_tok=-1, k_batch=2, v_tok=3, v_batch=4,
+                o_tok=5, o_batch=6, q_pos0=8, ctx_keys=9, chain_start=10, kv_batch=11, rope_rows_per_table=12,
+                rope_row0=13, rope_table_stride=14, rel_buckets=15, bias_head=16, bias_row=17)
+    for over in ({}, {"n_q": 1 << 33, "heads": -(1 << 31) - 1}, {"scale": 1e300}):
+        kw = dict(dict(ints, scale=0.5), **over)
+        a = ta.make_args(q=q, k=q, v=q, o=q, mask=ta.Mask.CAUSAL, key_valid=kv, rope_cos=q, rope_sin=q, bias=q, **kw)
+        b = ta.AttnArgs()
+        b.dtype, b.mask, b.head_dim, b.rope_half = 0, 2, 64, 32
+        for f in ("q", "k", "v", "o", "bias", "rope_cos", "rope_sin"):
+            setattr(b, f, q.ctypes.data)
+        b.key_valid = kv.ctypes.data
+        for f, value in kw.items():
+            setattr(b, f, value)
+        assert bytes(a) == bytes(b)

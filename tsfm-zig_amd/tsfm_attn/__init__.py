@@ -30,6 +30,7 @@ import enum
 import math
 import os
 import pathlib
+import struct
 from dataclasses import dataclass
 from typing import Any, Optional, Sequence
 
@@ -166,6 +167,13 @@ class AttnArgs(ctypes.Structure):
         ("rope_table_stride", ctypes.c_int64),
         ("stream", ctypes.c_void_p),
     ]
+
+
+# The argument block as one struct.pack: the C layout from the field types (native sizes and alignment).
+# Setting 43 ctypes fields one by one cost more host time than a small call's kernel takes.
+_ATTN_PACK = struct.Struct("@" + "".join({ctypes.c_int32: "i", ctypes.c_uint32: "I", ctypes.c_float: "f",
+                                          ctypes.c_int64: "q", ctypes.c_void_p: "P"}[t] for _, t in AttnArgs._fields_))
+assert _ATTN_PACK.size == ctypes.sizeof(AttnArgs)
 
 
 _lib: Optional[ctypes.CDLL] = None
@@ -531,10 +539,11 @@ def _ptr(x: Any) -> Optional[int]:
     """Address of a numpy array, a torch tensor, or an int; None stays None."""
     if x is None:
         return None
+    data_ptr = getattr(x, "data_ptr", None)
+    if data_ptr is not None:
+        return data_ptr()
     if isinstance(x, int):
         return x
-    if hasattr(x, "data_ptr"):
-        return x.data_ptr()
     if hasattr(x, "ctypes"):
         if not x.flags["C_CONTIGUOUS"]:
             raise ValueError("numpy arrays passed to tsfm_attn must be C-contiguous")
@@ -543,18 +552,28 @@ def _ptr(x: Any) -> Optional[int]:
 
 
 def _is_device(x: Any) -> bool:
-    return hasattr(x, "is_cuda") and bool(x.is_cuda)
+    return bool(getattr(x, "is_cuda", False))
+
+
+_DTYPE_CODES: dict = {}  # dtype object -> code, filled as dtypes are met (a handful)
 
 
 def _dtype_code(x: Any) -> int:
-    name = str(getattr(x, "dtype", "float32"))
+    dt = getattr(x, "dtype", "float32")
+    code = _DTYPE_CODES.get(dt)
+    if code is not None:
+        return code
+    name = str(dt)
     if "bfloat16" in name:
-        return DTYPE_BF16
-    if "float16" in name:
-        return DTYPE_F16
-    if "float32" in name:
-        return DTYPE_F32
-    raise TypeError(f"unsupported element type {name}")
+        code = DTYPE_BF16
+    elif "float16" in name:
+        code = DTYPE_F16
+    elif "float32" in name:
+        code = DTYPE_F32
+    else:
+        raise TypeError(f"unsupported element type {name}")
+    _DTYPE_CODES[dt] = code
+    return code
 
 
 def _stream_of(x: Any, stream: Any) -> Optional[int]:
@@ -563,6 +582,9 @@ def _stream_of(x: Any, stream: Any) -> Optional[int]:
     if _is_device(x):
         import torch  # device-pointer calls run on torch's current stream by default
 
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # without building a Stream object
+        if raw is not None:
+            return int(raw(x.get_device()))
         return int(torch.cuda.current_stream(x.device).cuda_stream)
     return None
 
@@ -620,25 +642,19 @@ def make_args(
 ) -> AttnArgs:
     """Build ``tsfm_attn_args``; device mode is chosen when q is a device tensor."""
     device = _is_device(q)
-    a = AttnArgs()
-    a.dtype = _dtype_code(q) if dtype is None else dtype
-    a.mask = int(mask)
-    a.batch, a.heads, a.n_q, a.n_k, a.head_dim = batch, heads, n_q, n_k, head_dim
-    a.q_pos0, a.ctx_keys, a.chain_start = q_pos0, ctx_keys, chain_start
-    a.scale = float(scale)
-    a.flags = DEVICE_PTRS if device else 0
-    a.q, a.q_tok, a.q_batch = _ptr(q), q_tok, q_batch
-    a.k, a.k_tok, a.k_batch = _ptr(k), k_tok, k_batch
-    a.v, a.v_tok, a.v_batch = _ptr(v), v_tok, v_batch
-    a.o, a.o_tok, a.o_batch = _ptr(o), o_tok, o_batch
-    a.key_valid, a.kv_batch = _ptr(key_valid), kv_batch
-    a.bias, a.bias_head, a.bias_row = _ptr(bias), bias_head, bias_row
-    a.rel_table, a.rel_bucket, a.rel_buckets = _ptr(rel_table), _ptr(rel_bucket), rel_buckets
-    a.rope_cos, a.rope_sin = _ptr(rope_cos), _ptr(rope_sin)
-    a.rope_half = head_dim // 2 if rope_cos is not None else 0
-    a.rope_rows_per_table, a.rope_row0, a.rope_table_stride = rope_rows_per_table, rope_row0, rope_table_stride
-    a.stream = _stream_of(q, stream) if device else None
-    return a
+    vals = (
+        _dtype_code(q) if dtype is None else dtype, int(mask), batch, heads, n_q, n_k, head_dim, q_pos0, ctx_keys,
+        chain_start, float(scale), DEVICE_PTRS if device else 0,
+        _ptr(q) or 0, q_tok, q_batch, _ptr(k) or 0, k_tok, k_batch, _ptr(v) or 0, v_tok, v_batch,
+        _ptr(o) or 0, o_tok, o_batch, _ptr(key_valid) or 0, kv_batch, _ptr(bias) or 0, bias_head, bias_row,
+        _ptr(rel_table) or 0, _ptr(rel_bucket) or 0, rel_buckets, _ptr(rope_cos) or 0, _ptr(rope_sin) or 0,
+        head_dim // 2 if rope_cos is not None else 0, rope_rows_per_table, rope_row0, rope_table_stride,
+        (_stream_of(q, stream) or 0) if device else 0,
+    )
+    try:
+        return AttnArgs.from_buffer_copy(_ATTN_PACK.pack(*vals))
+    except (struct.error, OverflowError):  # a value past its field: ctypes' own conversion
+        return AttnArgs(*vals)
 
 
 def _flat_view(x: Any, offset: int) -> Any:
