@@ -936,11 +936,20 @@ hipError_t encode_on(const tsfm_chronos2_encode_args* a, float* x, const uint8_t
         return fused ? tsfm::launch_rms_norm_planes(x, d, xn_pl, scale, R, D, a->eps, s)
                      : tsfm::launch_rms_norm(x, d, xn, d, scale, R, D, a->eps, s);
     };
+    // A residual product into x and the next row norm of x: without pre-split operands in one call (the
+    // norm rides on the sum of a split reduction, a launch fewer, the same bits).
+    auto residual_norm = [&](const float* in, int in_w, const float* w, const float* scale, float* out,
+                             const void* in_pl) {
+        if (!fused) return linear_norm_on(in, in_w, w, D, in_w, x, d, R, tsfm::kEpiResidual, x, scale, out, d, a->eps, s);
+        const hipError_t e1 = linear_on(in, in_w, w, D, in_w, x, d, R, tsfm::kEpiResidual, x, s, nullptr, in_pl);
+        if (e1 != hipSuccess || out != xn) return e1;
+        return norm(scale);
+    };
     hipError_t e = hipSuccess;
+    if (a->n_layers > 0) e = norm(layers[0].time_norm);
     for (int l = 0; l < a->n_layers && e == hipSuccess; l++) {
         const tsfm_chronos2_layer& ly = layers[l];
         // time attention
-        if ((e = norm(ly.time_norm)) != hipSuccess) break;
         tsfm::ProjParams p{};
         p.x = xn; p.x_tok = d; p.w0 = ly.time_q; p.w1 = ly.time_k; p.w2 = ly.time_v; p.w_ld = d;
         p.alpha = 1.f; p.epi = tsfm::kEpiNone;
@@ -957,25 +966,24 @@ hipError_t encode_on(const tsfm_chronos2_encode_args* a, float* x, const uint8_t
         ap.B = a->batch; ap.H = a->heads; ap.n_q = a->seq; ap.n_k = a->seq; ap.scale = a->scale;
         const int mask = a->keys_all_valid ? TSFM_MASK_FULL : TSFM_MASK_KEYS_ADDITIVE;  // Mask.pick(false, all, true)
         if ((e = tsfm::launch_attn_f32(ap, mask, tsfm::BIAS_NONE, false, s)) != hipSuccess) break;
-        if ((e = linear_on(ab, d, ly.time_o, D, D, x, d, R, tsfm::kEpiResidual, x, s)) != hipSuccess) break;
+        if ((e = residual_norm(ab, D, ly.time_o, ly.group_norm, xn, nullptr)) != hipSuccess) break;
         // group attention with singleton groups
-        if ((e = norm(ly.group_norm)) != hipSuccess) break;
         if ((e = linear_on(xn, d, ly.group_v, D, D, v, d, R, tsfm::kEpiNone, nullptr, s, nullptr,
                            fused ? xn_pl : nullptr, fused ? v_pl : nullptr)) != hipSuccess)
             break;
-        if ((e = linear_on(v, d, ly.group_o, D, D, x, d, R, tsfm::kEpiResidual, x, s, nullptr,
-                           fused ? v_pl : nullptr)) != hipSuccess)
-            break;
+        if ((e = residual_norm(v, D, ly.group_o, ly.mlp_norm, xn, v_pl)) != hipSuccess) break;
         // MLP
-        if ((e = norm(ly.mlp_norm)) != hipSuccess) break;
         if ((e = linear_on(xn, d, ly.mlp_wi, F, D, h, F, R, tsfm::kEpiRelu, nullptr, s, nullptr,
                            fused ? xn_pl : nullptr, fused ? h_pl : nullptr)) != hipSuccess)
             break;
-        if ((e = linear_on(h, F, ly.mlp_wo, D, F, x, d, R, tsfm::kEpiResidual, x, s, nullptr,
-                           fused ? h_pl : nullptr)) != hipSuccess)
+        // then the next layer's first norm, or the final one (in place)
+        const bool last = l + 1 == a->n_layers;
+        if ((e = residual_norm(h, F, ly.mlp_wo, last ? final_norm : layers[l + 1].time_norm, last ? x : xn, h_pl)) !=
+            hipSuccess)
             break;
     }
-    if (e == hipSuccess) e = tsfm::launch_rms_norm(x, d, x, d, final_norm, R, D, a->eps, s);
+    if (e == hipSuccess && (fused || a->n_layers == 0))
+        e = tsfm::launch_rms_norm(x, d, x, d, final_norm, R, D, a->eps, s);
     return e;
 }
 
