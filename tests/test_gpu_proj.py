@@ -371,3 +371,39 @@ def test_presplit_product_back_to_back_launches_agree(ta, gpu_ready):
     for outs in runs[1:]:
         for got, first in zip(outs, runs[0]):
             assert torch.equal(got.view(torch.int32), first.view(torch.int32))
+
+
+@pytest.mark.parametrize("b,seq,d,nh", [(12, 125, 768, 12), (20, 130, 512, 5), (20, 126, 512, 5), (16, 128, 512, 6),
+                                        (3, 1365, 768, 4)])
+def test_tile_choice_between_the_kernels(ta, gpu_ready, b, seq, d, nh):
+    """Products around the rules of tile and operand form: 216 tiles of 128 x 128 split inside the
+    product, 168 and 160 on pre-split operands over 2600 and 2520 rows, and 2048 and 4095 rows of at
+    least 2^30 multiply-adds: tsfm_qkv_project (operand workspace) and tsfm_qkv_project_noalloc (none)
+    give the same bits, within the bar of float64."""
+    import torch
+
+    tokens, inner = b * seq, nh * 64
+    rng = np.random.default_rng(tokens)
+    x = rng.standard_normal((tokens, d)).astype(np.float32)
+    ws = _weights(rng, inner, d, 3)
+    ang = np.outer(np.arange(seq), 10000.0 ** (-np.arange(32) / 32))
+    cos_t, sin_t = np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
+    dev = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, *ws, cos_t, sin_t)]
+    outs = []
+    for fn in (ta.qkv_project, ta.qkv_project_noalloc):
+        y = [torch.full((tokens, inner), -3.0, device="cuda") for _ in range(3)]
+        a = ta.ProjArgs(dtype=ta.DTYPE_F32, out_dtype=ta.DTYPE_F32, batch=b, seq=seq, d_in=d, heads=nh, head_dim=64,
+                        flags=ta.DEVICE_PTRS, rope_half=32, x=dev[0].data_ptr(), x_tok=d, w_q=dev[1].data_ptr(),
+                        w_k=dev[2].data_ptr(), w_v=dev[3].data_ptr(), q=y[0].data_ptr(), q_tok=inner,
+                        k=y[1].data_ptr(), k_tok=inner, v=y[2].data_ptr(), v_tok=inner, rope_cos=dev[4].data_ptr(),
+                        rope_sin=dev[5].data_ptr(), stream=0)
+        assert fn(a) == ta.OK, ta.last_error()
+        torch.cuda.synchronize()
+        outs.append([t.cpu().numpy() for t in y])
+    for pre, own in zip(*outs):
+        np.testing.assert_array_equal(pre, own)
+    for i, w in enumerate(ws):
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+        if i < 2:
+            want = _ref.rope_f64(want, cos_t, sin_t, seq, nh)
+        assert _ref.scaled_err(outs[0][i], want) <= TOL
