@@ -109,3 +109,17 @@ def test_noalloc_holds_the_largest_split_partials(ta, gpu_ready):
     got = _run(torch, ta, lib.tsfm_qkv_project_noalloc, c)
     for g, w_ in zip(got, want):
         assert np.array_equal(g, w_)
+
+
+@pytest.mark.parametrize("tokens,nh", [(448, 19), (448, 20), (64, 139), (64, 140)])
+def test_noalloc_at_the_split_rule_edge(ta, gpu_ready, tokens, nh):
+    """399 and 417 tiles of 64 x 64 split two ways (the rule aims at about 420 workgroups), 420 run
+    unsplit: the array's partials and the entry point's workspace give the same bits."""
+    import torch
+
+    lib = _lib(ta)
+    c = _case(torch, tokens + nh, tokens, 256, nh)
+    want = _run(torch, ta, lib.tsfm_qkv_project, c)
+    got = _run(torch, ta, lib.tsfm_qkv_project_noalloc, c)
+    for g, w_ in zip(got, want):
+        assert np.array_equal(g, w_)

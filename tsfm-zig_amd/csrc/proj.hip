@@ -1178,6 +1178,7 @@ bool proj_fuses_input_norm(int64_t tokens, int64_t d_in) {
     return tokens > 0 && tokens <= kSkinnyTokens && d_in > 0 && d_in <= kSkinnyMaxIn && d_in % 16 == 0;
 }
 
+constexpr int64_t kSplitBlocks = 420;
 size_t proj_split_bytes(ProjParams& p) {
     p.m_tiles = (p.tokens + BM - 1) / BM;
     p.n_tiles = (p.width * p.n_out + BN - 1) / BN;
@@ -1187,17 +1188,19 @@ size_t proj_split_bytes(ProjParams& p) {
     p.split_steps = steps;
     p.partial = nullptr;
     if (p.x_pre != nullptr || p.y_planes != nullptr || p.w_pre != nullptr) return 0;  // pre-split operands: never split
-    // f32 outputs, no RoPE; several outputs only without an epilogue; at most half a launch of
-    // tiles (four workgroups per CU), and at least 16 steps to share out.
-    if (!((p.n_out == 1 || p.epi == kEpiNone) && p.rope_cos == nullptr && p.out_dtype == 0 && blocks < 512 &&
+    // f32 outputs, no RoPE; several outputs only without an epilogue; fewer tiles than kSplitBlocks,
+    // and at least 16 steps to share out.
+    if (!((p.n_out == 1 || p.epi == kEpiNone) && p.rope_cos == nullptr && p.out_dtype == 0 && blocks < kSplitBlocks &&
           steps >= 16) ||
         skinny(p))
         return 0;
-    // About 512 workgroups (two per CU): more splits of these short reductions cost more in
-    // partial traffic and per-workgroup start-up than they gain in parallelism (measured on the
-    // Chronos-Bolt-small forecast: 1.160 ms for about 1024, 1.106 ms for about 512, 1.185 ms for
-    // at most two splits).
-    int s = (int)std::min<int64_t>((512 + blocks - 1) / blocks, std::min(steps / 8, 16));
+    // About kSplitBlocks workgroups: each split costs its start, its partial sums' trip through memory and
+    // the longer sum afterwards (half of an 18 us launch of 576 workgroups), so a product splits only
+    // while the CUs have fewer than about one and a half workgroups each. Whole calls in us, aiming at
+    // 360 / 420 / 470 / 512 workgroups: Chronos-2 layers of 545 rows 434 / 432 / 454 / 466, the
+    // Chronos-Bolt-small forecast 971 / 936 / 940 / 948, Chronos-Bolt-base layers of 528 rows 467 / 464 /
+    // 490 / 492, of 1056 rows 706 / 693 / 691 / 693.
+    int s = (int)std::min<int64_t>((kSplitBlocks + blocks - 1) / blocks, std::min(steps / 8, 16));
     if (s < 2) return 0;
     int per = (steps + s - 1) / s;
     if (p.d_in % X3_BK == 0) per += per & 1;  // whole 32-index steps for the bf16x3 kernel
@@ -1205,7 +1208,7 @@ size_t proj_split_bytes(ProjParams& p) {
     if (s < 2) return 0;
     p.splits = s;
     p.split_steps = per;
-    // s * blocks <= 512 + blocks - 1 < 1536 and tokens * width <= blocks * BM * BN, so the partials
+    // s * blocks <= kSplitBlocks + blocks - 1 < 1536 and tokens * width <= blocks * BM * BN, so the partials
     // always fit kSplitWorkspaceBytes.
     return (size_t)s * p.tokens * p.width * p.n_out * sizeof(float);
 }
