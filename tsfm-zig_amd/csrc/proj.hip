@@ -914,17 +914,6 @@ __global__ __launch_bounds__(64 * SKW) void proj_skinny(ProjParams p) {
     const int r = lane & 15, kq = 4 * (lane >> 4);
     const float* const xr = p.x + (int64_t)min(r, p.tokens - 1) * p.x_tok + kq;
     const bool in_norm = p.in_norm_scale != nullptr;  // uniform
-    if (in_norm) {
-        // Wave w: the norm of token row w (clamped as the loads are), with rms_norm_rows' lane
-        // mapping and order, so the normalised inputs have its bits.
-        const float* const xw = p.x + (int64_t)min(wave, p.tokens - 1) * p.x_tok;
-        float ss = 0.f;
-        for (int i = 4 * lane; i < p.d_in; i += 256) ss = sumsq4(ss, ld4(xw + i));
-        const float inv = rms_inv(ss, p.d_in, p.in_norm_eps);
-        if (lane == 0) inv_s[wave] = inv;
-        __syncthreads();
-    }
-    const float inv_r = in_norm ? inv_s[r] : 1.f;
     const float* const sr = in_norm ? p.in_norm_scale + kq : nullptr;
     const float* wr;
     {  // weight row of the lane's column (clamped past the last column)
@@ -933,22 +922,55 @@ __global__ __launch_bounds__(64 * SKW) void proj_skinny(ProjParams p) {
         const float* w = sel == 0 ? p.w0 : sel == 1 ? p.w1 : sel == 2 ? p.w2 : p.w3;
         wr = w + (int64_t)(n - sel * p.width) * p.w_ld + kq;
     }
+    // Everything the workgroup reads is issued before anything waits: the wave's norm row, its first
+    // units, and (the threads that finish) the epilogue's operands.
+    f32x4 xs[SKB], ws[SKB], ss4[SKB];
+    auto fetch = [&](int b0) {
+        const int nb = min(SKB, u1 - b0);
+#pragma unroll
+        for (int i = 0; i < SKB; i++) {
+            if (i < nb) {
+                ws[i] = ld4(wr + 16 * (b0 + i));
+                xs[i] = ld4(xr + 16 * (b0 + i));
+                if (in_norm) ss4[i] = ld4(sr + 16 * (b0 + i));
+            }
+        }
+    };
+    f32x4 nr[kSkinnyMaxIn / 256];
+    if (in_norm) {
+        const float* const xw = p.x + (int64_t)min(wave, p.tokens - 1) * p.x_tok;
+#pragma unroll
+        for (int i = 0; i < kSkinnyMaxIn / 256; i++)
+            if (4 * lane + 256 * i < p.d_in) nr[i] = ld4(xw + 4 * lane + 256 * i);
+    }
+    fetch(u0);
+    const int m = tid >> 2, c4 = 4 * (tid & 3), c = tn * 16 + c4;
+    const bool finisher = tid < kSkinnyTokens * 4 && m < p.tokens && c < n_cols;
+    const int sel = c / p.width, col = c - sel * p.width;
+    f32x4 bias = {0.f, 0.f, 0.f, 0.f}, res = bias;
+    if (finisher && p.bias != nullptr) bias = ld4(p.bias + col);
+    if (finisher && p.epi == kEpiResidual) res = ld4(p.resid + (int64_t)m * p.resid_tok + col);
+    if (in_norm) {
+        // Wave w: the norm of token row w (clamped as the loads are), with rms_norm_rows' lane
+        // mapping and order, so the normalised inputs have its bits.
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < kSkinnyMaxIn / 256; i++)
+            if (4 * lane + 256 * i < p.d_in) ss = sumsq4(ss, nr[i]);
+        const float inv = rms_inv(ss, p.d_in, p.in_norm_eps);
+        if (lane == 0) inv_s[wave] = inv;
+        __syncthreads();
+    }
+    const float inv_r = in_norm ? inv_s[r] : 1.f;
     f32x4 tot = {0.f, 0.f, 0.f, 0.f}, chk = tot;
     int cu = 0;  // units done in the running chunk
     for (int b0 = u0; b0 < u1; b0 += SKB) {
         const int nb = min(SKB, u1 - b0);
-        f32x4 xs[SKB], ws[SKB];
-#pragma unroll
-        for (int i = 0; i < SKB; i++) {
-            if (i < nb) {
-                xs[i] = ld4(xr + 16 * (b0 + i));
-                ws[i] = ld4(wr + 16 * (b0 + i));
-            }
-        }
+        if (b0 > u0) fetch(b0);
         if (in_norm) {
 #pragma unroll
             for (int i = 0; i < SKB; i++)
-                if (i < nb) xs[i] = rms_apply(xs[i], inv_r, ld4(sr + 16 * (b0 + i)));
+                if (i < nb) xs[i] = rms_apply(xs[i], inv_r, ss4[i]);
         }
 #pragma unroll
         for (int i = 0; i < SKB; i++) {
@@ -966,12 +988,20 @@ __global__ __launch_bounds__(64 * SKW) void proj_skinny(ProjParams p) {
     // Lane l holds columns 4 (l >> 4) .. + 3 of token l & 15.
     st4(smem + (wave * kSkinnyTokens + r) * 16 + kq, tot);
     __syncthreads();
-    if (tid >= kSkinnyTokens * 4) return;
-    const int m = tid >> 2, c4 = 4 * (tid & 3), c = tn * 16 + c4;
-    if (m >= p.tokens || c >= n_cols) return;
-    f32x4 v = ld4(smem + m * 16 + c4);
-    for (int w = 1; w < SKW; w++) v = v + ld4(smem + (w * kSkinnyTokens + m) * 16 + c4);
-    finish4(p, m, c, v);
+    if (!finisher) return;
+    f32x4 part[SKW];
+#pragma unroll
+    for (int w = 0; w < SKW; w++) part[w] = ld4(smem + (w * kSkinnyTokens + m) * 16 + c4);
+    f32x4 v = part[0];
+#pragma unroll
+    for (int w = 1; w < SKW; w++) v = v + part[w];
+    // finish4 with its operands already read
+    if (p.alpha != 1.f) v *= p.alpha;
+    if (p.bias != nullptr) v = v + bias;
+    if (p.epi == kEpiResidual) v = res + v;
+    else v = epi_act(p.epi, v);
+    float* const y = static_cast<float*>(sel == 0 ? p.y0 : sel == 1 ? p.y1 : sel == 2 ? p.y2 : p.y3);
+    st4(y + out_offset(p, sel, m) + col, v);
 }
 
 }  // namespace
