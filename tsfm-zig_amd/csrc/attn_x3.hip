@@ -222,6 +222,10 @@ __global__ __launch_bounds__(XNT) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     // ---- the wave's queries: rotated, scaled (the scale is a power of two in every family, so
     //      (scale q) . k is the reference's alpha (q . k) bit for bit) and split ----
     if (BIAS == BIAS_REL) fill_rel_lut(lut_raw, p, h, tid, nt);
+    // With the T5 bias (rows of 129 in use) the first chunk's loads are in flight across the single-query
+    // pass: Chronos-Bolt 140.3 -> 138.4 us. The other forms load after it: held across it, the loads'
+    // registers spill (27 with RoPE: 427 -> 434 us at 577 keys, which has no such pass).
+    if constexpr (BIAS == BIAS_REL && !ROPE) load_chunk(0);
     if (thin && qt == q_tiles - 1) {
         // ---- the single query past the blocks (n_q = 32k + 1), in the workgroup of the last blocks,
         //      before the blocks' own work: each wave takes a slice of the keys from K / V in global
@@ -319,7 +323,7 @@ __global__ __launch_bounds__(XNT) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         }
 
     }
-    load_chunk(0);
+    if constexpr (BIAS != BIAS_REL || ROPE) load_chunk(0);
     u32x4 qf[3][4];  // [plane][k-step]: dims 16s + 8 hh .. +7 of query qi
     {
         f32x4 qa[4][2];
