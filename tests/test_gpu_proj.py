@@ -407,3 +407,25 @@ def test_tile_choice_between_the_kernels(ta, gpu_ready, b, seq, d, nh):
         if i < 2:
             want = _ref.rope_f64(want, cos_t, sin_t, seq, nh)
         assert _ref.scaled_err(outs[0][i], want) <= TOL
+
+
+@pytest.mark.parametrize("tokens", [1, 7, 8, 9, 16, 17])
+@pytest.mark.parametrize("d_in", [16, 48, 256, 1024, 2048, 2064, 3072, 3088])
+def test_few_rows_at_the_edges_of_their_kernel(ta, gpu_ready, tokens, d_in):
+    """Products of at most 16 rows and reductions up to 2048 (up to eight rows: 3072) run in one launch
+    of column tiles whose waves share the reduction; longer ones and 17 rows elsewhere. Against
+    float64 within the textbook bound of a float32 product."""
+    import torch
+
+    nh = 1
+    rng = np.random.default_rng(100 * tokens + d_in)
+    x = rng.standard_normal((tokens, d_in)).astype(np.float32)
+    ws = [rng.standard_normal((nh * 64, d_in)).astype(np.float32) for _ in range(3)]
+    dx, dw = torch.from_numpy(x).cuda(), [torch.from_numpy(w).cuda() for w in ws]
+    y = [torch.full((tokens, nh * 64), -3.0, device="cuda") for _ in range(3)]
+    assert ta.bolt_qkv_projection(dx, *dw, *y, 1, tokens, d_in, nh, 64) == ta.OK, ta.last_error()
+    torch.cuda.synchronize()
+    for got, w in zip(y, ws):
+        want = x.astype(np.float64) @ w.astype(np.float64).T
+        bound = d_in * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T)
+        assert (np.abs(got.cpu().numpy() - want) <= bound).all()

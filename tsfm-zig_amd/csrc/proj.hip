@@ -890,18 +890,22 @@ __global__ __launch_bounds__(256) void proj_reduce_norm(ProjParams p) {
 // RoPE. Such a product is a few MB of weights read once: it is bound by how many loads are in
 // flight, not by the matrix cores. A workgroup takes one 16-column tile of every token and its
 // sixteen waves split the reduction: wave w takes the 16-wide units [w U / 16, (w + 1) U / 16) of
-// U = d_in / 16 and issues the loads of up to SKB of them at once, straight from HBM/L2 into
+// U = d_in / 16 and issues the loads of SKB of them at once, straight from HBM/L2 into
 // registers in the matrix instruction's layout (lane l: row l & 15 of a 16-row block, indices
 // 4 (l >> 4) .. + 3 of the unit), then multiplies them, accumulating blockwise as qkv_proj does.
 // The sixteen 16 x 16 partials meet in LDS and are added in wave order, then the epilogue: one
 // launch where a split over workgroups would need a second one for the sums.
 constexpr int SKW = 16;  // waves of a workgroup
-constexpr int SKB = 8;   // units a wave has in flight
+constexpr int SKB = 2;   // units in a batch: a 1024-thread workgroup has 128 registers a lane, and eight
+                         // units with the norm's row in flight too spilled 32 of them
 constexpr int kSkinnyTokens = 16;
-// Longer reductions read more weight bytes per column tile than the few CUs of a 16-token launch
-// (one per 64 columns) pull in time; they split over workgroups instead (measured at d_in 2048:
-// 13 us in one launch, 7 + 4 us split and summed).
-constexpr int kSkinnyMaxIn = 1024;
+// The longest reductions it takes, and with the input norm (the norm's row is held in registers).
+// Longer ones read more weight bytes per column tile than the few CUs of the launch pull in time and
+// split over workgroups instead, whose sum costs a second launch. Whole Chronos-Bolt forecasts in us,
+// longest 1024 / 2048 / 3072: 16 series of d_ff 2048 917 / 908 / 918, of 3072 883 / 874 / 886; 4 series of
+// 3072 661 / 654 / 635, one 482 / 469 / 432, one of d_ff 2048 376 / 348 / 348.
+constexpr int kSkinnyNormIn = 1024;
+static int skinny_max_in(int64_t tokens) { return tokens <= 8 ? 3072 : 2048; }
 constexpr size_t kSkinnyLds = (size_t)SKW * kSkinnyTokens * 16 * sizeof(float);
 __global__ __launch_bounds__(64 * SKW) void proj_skinny(ProjParams p) {
     extern __shared__ __attribute__((aligned(16))) float smem[];  // [wave][token][16 columns]
@@ -936,11 +940,11 @@ __global__ __launch_bounds__(64 * SKW) void proj_skinny(ProjParams p) {
             }
         }
     };
-    f32x4 nr[kSkinnyMaxIn / 256];
+    f32x4 nr[kSkinnyNormIn / 256];
     if (in_norm) {
         const float* const xw = p.x + (int64_t)min(wave, p.tokens - 1) * p.x_tok;
 #pragma unroll
-        for (int i = 0; i < kSkinnyMaxIn / 256; i++)
+        for (int i = 0; i < kSkinnyNormIn / 256; i++)
             if (4 * lane + 256 * i < p.d_in) nr[i] = ld4(xw + 4 * lane + 256 * i);
     }
     fetch(u0);
@@ -955,7 +959,7 @@ __global__ __launch_bounds__(64 * SKW) void proj_skinny(ProjParams p) {
         // mapping and order, so the normalised inputs have its bits.
         float ss = 0.f;
 #pragma unroll
-        for (int i = 0; i < kSkinnyMaxIn / 256; i++)
+        for (int i = 0; i < kSkinnyNormIn / 256; i++)
             if (4 * lane + 256 * i < p.d_in) ss = sumsq4(ss, nr[i]);
         const float inv = rms_inv(ss, p.d_in, p.in_norm_eps);
         if (lane == 0) inv_s[wave] = inv;
@@ -1200,12 +1204,12 @@ static int proj_chunk(int units) {
 
 // Products the 16-token kernel takes (proj_skinny).
 static bool skinny(const ProjParams& p) {
-    return p.tokens <= kSkinnyTokens && p.d_in <= kSkinnyMaxIn && p.rope_cos == nullptr && p.out_dtype == 0 &&
+    return p.tokens <= kSkinnyTokens && p.d_in <= skinny_max_in(p.tokens) && p.rope_cos == nullptr && p.out_dtype == 0 &&
            p.x_pre == nullptr && p.y_planes == nullptr && p.w_pre == nullptr;
 }
 
 bool proj_fuses_input_norm(int64_t tokens, int64_t d_in) {
-    return tokens > 0 && tokens <= kSkinnyTokens && d_in > 0 && d_in <= kSkinnyMaxIn && d_in % 16 == 0;
+    return tokens > 0 && tokens <= kSkinnyTokens && d_in > 0 && d_in <= kSkinnyNormIn && d_in % 16 == 0;
 }
 
 constexpr int64_t kSplitBlocks = 420;
@@ -1258,7 +1262,8 @@ hipError_t launch_proj(const ProjParams& p0, hipStream_t stream) {
         return hipErrorInvalidValue;
     if ((int64_t)((p.tokens + BM - 1) / BM) * ((p.width * p.n_out + BN - 1) / BN) > 0x7fffffff)
         return hipErrorInvalidValue;
-    if (p.in_norm_scale != nullptr && !skinny(p)) return hipErrorInvalidValue;  // the 16-token kernel only
+    if (p.in_norm_scale != nullptr && (!skinny(p) || p.d_in > kSkinnyNormIn))
+        return hipErrorInvalidValue;  // the 16-token kernel only
     if (skinny(p)) {
         p.chunk = proj_chunk((p.d_in / 16 + SKW - 1) / SKW);
         hipLaunchKernelGGL(proj_skinny, dim3((unsigned)((p.width * p.n_out + 15) / 16)), dim3(64 * SKW), kSkinnyLds,
