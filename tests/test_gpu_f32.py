@@ -419,3 +419,64 @@ def test_short_rows_on_both_sides_of_the_kernel_choice(ta, gpu_ready, mask, n_q,
             allowed = _ref.allowed_matrix(mask, n_q, n_k, kv[b], **extra)
             want = _ref.naive_attend(q[b, :, sel], k[b, :, sel], v[b, :, sel], allowed, 0.125)
             assert _ref.scaled_err(got[b, :, sel], want) <= TOL, (B, b, h)
+
+
+@pytest.mark.parametrize("mask,n_q,n_k,form", [
+    (mask, n_q, n_k, form) for mask, n_q, n_k in ((0, 24, 24), (1, 64, 64), (1, 97, 97), (1, 129, 129), (0, 129, 129),
+                                                  (1, 144, 144), (2, 100, 100), (4, 80, 80), (4, 144, 144), (5, 32, 94))
+    for form in ("plain", "rope", "dense", "t5") if (mask, form) != (5, "t5")])  # (the T5 table has no query offset)
+def test_short_rows_with_infinite_and_huge_operands(ta, gpu_ready, mask, n_q, n_k, form):
+    """Rows of at most 144 keys give what f32 arithmetic gives on either kernel: an infinite K value
+    whose scores are all -inf leaves its key without weight, as a finite one past the largest bf16 (3.39e38)
+    does; such a V value gives finite outputs, an infinite one an infinite dim and no other. 516 rows of
+    one size, and 2."""
+    rng = np.random.default_rng(n_q + 1000 * mask)
+    H = 6
+    extra = dict(q_pos0=n_k - n_q) if mask >= 2 else {}
+    if mask == 5:
+        extra.update(ctx_keys=n_k - n_q, chain_start=n_k - n_q)
+    bias = None
+    if form == "dense":
+        bias = rng.standard_normal((H, n_q, n_k)).astype(np.float32)
+        extra.update(bias=bias, bias_head=n_q * n_k, bias_row=n_k)
+    if form == "t5":
+        table = rng.standard_normal((32, H)).astype(np.float32)
+        bucket = np.zeros(n_q + n_k - 1, np.int32)
+        assert ta.load().tsfm_t5_bucket_table(bucket.ctypes.data, n_q, n_k, 32, 128) == ta.OK
+        extra.update(rel_table=table, rel_bucket=bucket, rel_buckets=32)
+        rel = np.arange(n_k)[None, :] - np.arange(n_q)[:, None] + n_q - 1
+        bias = table[bucket[rel]].transpose(2, 0, 1)
+    if form == "rope":
+        ang = np.outer(np.arange(n_k), 10000.0 ** (-np.arange(32) / 32))
+        cos_t, sin_t = np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
+        extra.update(rope_cos=cos_t, rope_sin=sin_t)
+    key = 0 if mask in (2, 5) else n_k - 1 if n_k % 32 == 1 else n_k // 2
+    for kind in ("v_inf", "v_huge") + (() if form == "rope" else ("k_inf", "k_huge")):
+        for B in (86, 1):
+            heads = H if B > 1 else 2
+            q, k, v, kv = _inputs(n_q + B, B, heads, n_q, n_k)
+            q *= 0.125
+            kv[:, key] = 1
+            if kind[0] == "k":
+                q[:, :, ::64] = 1.0
+            bad = dict(v_inf=np.inf, v_huge=3.4e38, k_inf=-np.inf, k_huge=-3.4e38)[kind]
+            (k if kind[0] == "k" else v)[:, key, ::64] = bad
+            got = run_generic(ta, mask, q, k, v, kv, B, heads, n_q, n_k, 1.0,
+                              **{n: a[:heads] if n == "bias" else np.ascontiguousarray(a[:, :heads]) if n == "rel_table" else a
+                                 for n, a in extra.items()})
+            pos = {n: extra[n] for n in ("q_pos0", "ctx_keys", "chain_start") if n in extra}
+            for b, h in ((0, 0), (B // 2, 1), (B - 1, heads - 1)):
+                sel = slice(h * 64, h * 64 + 64)
+                qh, kh = q[b, :, sel].astype(np.float64), k[b, :, sel].astype(np.float64)
+                if form == "rope":
+                    p0 = pos.get("q_pos0", 0)
+                    qh = _ref.rope_f64(qh, cos_t[p0:p0 + n_q], sin_t[p0:p0 + n_q], n_q, 1)
+                    kh = _ref.rope_f64(kh, cos_t, sin_t, n_k, 1)
+                allowed = _ref.allowed_matrix(mask, n_q, n_k, kv[b], **pos)
+                with np.errstate(invalid="ignore"):
+                    want = _ref.naive_attend(qh, kh, v[b, :, sel], allowed, 1.0, None if bias is None else bias[h])
+                g = got[b, :, sel]
+                fin = np.isfinite(want)  # (a causal query of the -inf key alone has no weights: NaN)
+                assert np.array_equal(g[~fin], want[~fin].astype(np.float32), equal_nan=True), (kind, B, b, h)
+                assert np.isfinite(g[fin]).all(), (kind, B, b, h)
+                assert _ref.scaled_err(g[fin], want[fin]) <= TOL, (kind, B, b, h)

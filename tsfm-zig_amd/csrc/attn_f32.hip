@@ -416,7 +416,6 @@ __device__ __forceinline__ void store_o(const QBlock& w, float* O, const Params&
 constexpr int RNW = 9;                  // waves per workgroup
 constexpr int RNT = 64 * RNW;           // threads
 constexpr int RQT = 16 * RNW;           // queries per workgroup (144)
-constexpr int kResidentKeys = 144;      // longest row the resident kernel takes
 constexpr int RNK = 32;                 // keys per tile of the resident loop
 constexpr int RKIT = (kResidentKeys * 8 + RNT - 1) / RNT;   // K staging items per thread
 constexpr int RVIT = (kResidentKeys * 8 + RNT - 1) / RNT;   // V staging items per thread

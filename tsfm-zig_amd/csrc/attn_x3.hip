@@ -103,7 +103,88 @@ __device__ __forceinline__ float pair_sum(float x) {
     return __uint_as_float(a[0]) + __uint_as_float(a[1]);
 }
 
+// One query in plain f32 by its wave: its normalised output, dim `lane` of it in each lane. For rows of at
+// most kResidentKeys keys whose matrix result is not finite: the split has no form for an infinity, nor for
+// a value that rounds past the largest bf16 (inf - inf), so such an operand makes the row's scores or
+// outputs NaN where f32 arithmetic may not: a score of -inf has weight 0, an infinite V gives infinite
+// outputs. Same bias, mask and weights as the resident f32 kernel, which other calls of such rows run on;
+// the keys it weighs with 0 past the query's own range (whole 16-key blocks) included. scr: kRedoScratch
+// floats of the wave's own. Only the check runs when the results are finite: 32 additions a wave (256 x 12
+// rows of 129 with the T5 bias: 142.4 us with it, 142.0 without).
+constexpr int kRedoScratch = kHeadDim + (kResidentKeys + 63) / 64 * 64;
 template <int MASK, int BIAS, bool ROPE>
+__device__ __forceinline__ float redo_query(const float* lut, float* scr, int b, int h, int qi, int lane) {
+#pragma clang fp contract(off)
+    // The kernel's arguments read again, through a pointer the optimiser cannot see through: kept from the
+    // top of the kernel for this path, they would take up to thirty scalar registers through its loops.
+    uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    const Params& p = *(const Params*)(const __attribute__((address_space(4))) Params*)args;
+    const float* const Q = static_cast<const float*>(p.q) + b * p.q_batch + h * kHeadDim;
+    const float* const K = static_cast<const float*>(p.k) + b * p.k_batch + h * kHeadDim;
+    const float* const V = static_cast<const float*>(p.v) + b * p.v_batch + h * kHeadDim;
+    const int rope_tab = p.rope_rows_per_table > 0 ? (p.rope_row0 + b) / p.rope_rows_per_table : 0;
+    const float* const RC = ROPE ? p.rope_cos + rope_tab * p.rope_table_stride : nullptr;
+    const float* const RS = ROPE ? p.rope_sin + rope_tab * p.rope_table_stride : nullptr;
+    const int n_valid = mask_reads_valid<MASK>() ? valid_len<MASK>(p.n_k, p.ctx_keys) : 0;
+    const int qpos = p.q_pos0 + qi;
+    const int kend =
+        min(p.n_k, (key_end_for<MASK>(p.q_pos0 + min(p.n_q - 1, qi | 15), p.n_k, p.ctx_keys) + 15) & ~15);
+    if (lane < 32) {
+        float x1 = Q[(int64_t)qi * p.q_tok + lane], x2 = Q[(int64_t)qi * p.q_tok + lane + 32];
+        if (ROPE) {  // nn.ropeHalf, src/core/nn.zig:453-460
+            const float c = RC[(int64_t)qpos * 32 + lane], sn = RS[(int64_t)qpos * 32 + lane];
+            const float y1 = x1 * c - x2 * sn, y2 = x2 * c + x1 * sn;
+            x1 = y1;
+            x2 = y2;
+        }
+        scr[lane] = x1 * p.scale;
+        scr[lane + 32] = x2 * p.scale;
+    }
+    __builtin_amdgcn_wave_barrier();  // LDS keeps a wave's accesses in order
+    float* const w = scr + kHeadDim;
+    float m = kNegInf;
+#pragma unroll 1
+    for (int key = lane; key < kend; key += 64) {
+        const float* kr = K + (int64_t)key * p.k_tok;
+        float x = 0.f;
+#pragma unroll 1
+        for (int c = 0; c < 8; c++) {
+            f32x4 lo = ld4(kr + 4 * c), hi = ld4(kr + 32 + 4 * c);
+            if (ROPE) rope4(lo, hi, ld4(RC + (int64_t)key * 32 + 4 * c), ld4(RS + (int64_t)key * 32 + 4 * c));
+            const f32x4 qa = ld4(scr + 4 * c), qb = ld4(scr + 32 + 4 * c);
+            for (int i = 0; i < 4; i++) x = __builtin_fmaf(qb[i], hi[i], __builtin_fmaf(qa[i], lo[i], x));
+        }
+        if (BIAS == BIAS_REL) x = x + lut[key - qi + p.n_q - 1];
+        if (BIAS == BIAS_DENSE) x = x + p.bias[h * p.bias_head + (int64_t)qi * p.bias_row + key];
+        const bool valid = !mask_reads_valid<MASK>() || (key < n_valid && p.key_valid[b * p.kv_batch + key] != 0);
+        x = masked<MASK>(x, key_term<MASK>(key, p.n_k, valid, p.ctx_keys), key, qpos, p.n_k, p.chain_start);
+        w[key] = x;
+        m = fmaxf(m, x);
+    }
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    const float m_use = m == kNegInf ? 0.f : m;
+    const bool big = m_use < -1e30f;
+    const float shift = big ? m_use : 0.f, ml = big ? 0.f : m_use * kLog2e;
+    float l = 0.f;
+#pragma unroll 1
+    for (int key = lane; key < kend; key += 64) {
+        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(w[key] - shift, kLog2e, -ml));
+        w[key] = e;
+        l += e;
+    }
+    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+    __builtin_amdgcn_wave_barrier();
+    float out = 0.f;
+#pragma unroll 4
+    for (int key = 0; key < kend; key++) out = __builtin_fmaf(w[key], V[(int64_t)key * p.v_tok + lane], out);
+    return out * (1.0f / l);
+}
+
+// SHORT: rows of at most kResidentKeys keys, whose results are checked (redo_query). A kernel of its own:
+// with the check in one kernel for all, the long rows' registers are laid out worse (577 keys with RoPE:
+// 442 us, 437 apart).
+template <int MASK, int BIAS, bool ROPE, bool SHORT>
 __global__ __launch_bounds__(XNT) __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_fwd_x3(Params p) {
     __shared__ __attribute__((aligned(16))) XStage stage[2];
     extern __shared__ float lut_raw[];  // the T5 table (n_q + n_k - 1 + margins), sized at launch
@@ -226,6 +307,7 @@ __global__ __launch_bounds__(XNT) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
     // pass: Chronos-Bolt 140.3 -> 138.4 us. The other forms load after it: held across it, the loads'
     // registers spill (27 with RoPE: 427 -> 434 us at 577 keys, which has no such pass).
     if constexpr (BIAS == BIAS_REL && !ROPE) load_chunk(0);
+    [[maybe_unused]] bool thin_odd = false;  // wave 0: the single query's result is not finite (redone at the end)
     if (thin && qt == q_tiles - 1) {
         // ---- the single query past the blocks (n_q = 32k + 1), in the workgroup of the last blocks,
         //      before the blocks' own work: each wave takes a slice of the keys from K / V in global
@@ -319,7 +401,9 @@ __global__ __launch_bounds__(XNT) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             L = L + tml[w][1] * sw;
             acc = acc + tw[w][lane] * sw;
         }
-        O[(int64_t)qn * p.o_tok + lane] = acc / L;
+        const float y = acc / L;
+        if constexpr (SHORT) thin_odd = __ballot(!(fabsf(y) <= kFltMax)) != 0;
+        O[(int64_t)qn * p.o_tok + lane] = y;
         }
 
     }
@@ -576,6 +660,24 @@ __global__ __launch_bounds__(XNT) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                 *reinterpret_cast<f32x4*>(ob + ql * kHeadDim + 4 * (c ^ (ql & 15))) =
                     f32x4{o[db][4 * g4], o[db][4 * g4 + 1], o[db][4 * g4 + 2], o[db][4 * g4 + 3]} * inv;
             }
+        if constexpr (SHORT) {
+            // Not finite if a value of the lane's is not (or if the sum of finite ones overflows: redone alike).
+            f32x4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 32; r++) part[r & 3] += o[r >> 4][r & 15];
+            const float sum = (part[0] + part[1]) + (part[2] + part[3]);
+            const uint64_t odd = __ballot(ql < wave_nq && !(fabsf(sum) <= kFltMax));
+            uint64_t todo = ((odd | odd >> 32) & 0xffffffffu) | (uint64_t)thin_odd << 32;  // bit 32: the single query
+            for (; todo != 0; todo &= todo - 1) {
+                const int r = __builtin_ctzll(todo), q = r < XQ ? wq0 + r : p.n_q - 1;
+                float* const scr = reinterpret_cast<float*>(&stage[0]) + XMAXW * XQ * kHeadDim + wave * kRedoScratch;
+                const float y = redo_query<MASK, BIAS, ROPE>(lut, scr, b, h, q, lane);
+                if (r < XQ) ob[r * kHeadDim + 4 * ((lane >> 2) ^ (r & 15)) + (lane & 3)] = y;
+                else O[(int64_t)q * p.o_tok + lane] = y;
+            }
+            static_assert((XMAXW * (XQ * kHeadDim + kRedoScratch)) * sizeof(float) <= sizeof(stage),
+                          "the rows and the scratch fit the stages");
+        }
         const int c = lane & 15;
 #pragma unroll
         for (int k = 0; k < XQ / 4; k++) {
@@ -597,7 +699,8 @@ hipError_t launch_one(const Params& p, hipStream_t stream) {
     const int64_t blocks = (int64_t)p.B * p.H * ((n_main + nw * XQ - 1) / (nw * XQ));
     if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
     const size_t lut_bytes = BIAS == BIAS_REL ? (size_t)(p.n_q + p.n_k - 1 + 2 * kLutPad) * sizeof(float) : 0;
-    hipLaunchKernelGGL((attn_fwd_x3<MASK, BIAS, ROPE>), dim3((unsigned)blocks), dim3(64 * nw), lut_bytes, stream, p);
+    const auto kernel = p.n_k <= kResidentKeys ? attn_fwd_x3<MASK, BIAS, ROPE, true> : attn_fwd_x3<MASK, BIAS, ROPE, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(64 * nw), lut_bytes, stream, p);
     return hipGetLastError();
 }
 

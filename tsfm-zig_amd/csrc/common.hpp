@@ -43,6 +43,9 @@ enum BiasKind : int { BIAS_NONE = 0, BIAS_DENSE = 1, BIAS_REL = 2 };
 // Longest T5 relative-offset table kept in LDS (n_q + n_k - 1 entries).
 constexpr int kRelMax = 2048;
 
+// Longest row (keys) the f32 kernel with resident keys takes (attn_f32.hip).
+constexpr int kResidentKeys = 144;
+
 // Kernel arguments, by value. Strides are in elements.
 struct Params {
     const void* q;
