@@ -480,3 +480,46 @@ def test_short_rows_with_infinite_and_huge_operands(ta, gpu_ready, mask, n_q, n_
                 assert np.array_equal(g[~fin], want[~fin].astype(np.float32), equal_nan=True), (kind, B, b, h)
                 assert np.isfinite(g[fin]).all(), (kind, B, b, h)
                 assert _ref.scaled_err(g[fin], want[fin]) <= TOL, (kind, B, b, h)
+
+
+@pytest.mark.parametrize("mask,n_q,n_k,form", [
+    (mask, n_q, n_k, form) for mask, n_q, n_k in ((1, 16, 16), (1, 37, 37), (1, 66, 66), (0, 69, 69), (1, 128, 128),
+                                                  (1, 129, 129), (1, 130, 130), (0, 144, 144), (4, 24, 24), (4, 80, 80),
+                                                  (4, 144, 144), (5, 40, 80), (5, 72, 144))
+    for form in ("rope", "dense", "t5", "t5+rope") if mask != 5 or "t5" not in form])  # (the T5 table has no query offset)
+def test_short_rows_of_every_form_on_both_kernels(ta, gpu_ready, mask, n_q, n_k, form):
+    """The forms the choice of kernel for rows of at most 144 keys tells apart (a RoPE table, a dense bias, the T5
+    table, hard and soft key masks), at row counts that run on one kernel or the other, against float64."""
+    rng = np.random.default_rng(n_q + 1000 * mask)
+    H = 6
+    extra = dict(q_pos0=n_k - n_q, ctx_keys=n_k - n_q, chain_start=n_k - n_q) if mask == 5 else {}
+    pos = dict(extra)
+    bias, ropes = None, {}
+    if form == "dense":
+        bias = rng.standard_normal((H, n_q, n_k)).astype(np.float32)
+    if "t5" in form:
+        table = rng.standard_normal((32, H)).astype(np.float32)
+        bucket = np.zeros(n_q + n_k - 1, np.int32)
+        assert ta.load().tsfm_t5_bucket_table(bucket.ctypes.data, n_q, n_k, 32, 128) == ta.OK
+        bias = table[bucket[np.arange(n_k)[None, :] - np.arange(n_q)[:, None] + n_q - 1]].transpose(2, 0, 1)
+    if "rope" in form:
+        ang = np.outer(np.arange(n_k), 10000.0 ** (-np.arange(32) / 32))
+        ropes = dict(rope_cos=np.cos(ang).astype(np.float32), rope_sin=np.sin(ang).astype(np.float32))
+    for B in (86, 84, 43, 21, 1):
+        heads = H if B > 1 else 2
+        q, k, v, kv = _inputs(n_q + B, B, heads, n_q, n_k)
+        if form == "dense":
+            extra.update(bias=bias[:heads].copy(), bias_head=n_q * n_k, bias_row=n_k)
+        if "t5" in form:
+            extra.update(rel_table=np.ascontiguousarray(table[:, :heads]), rel_bucket=bucket, rel_buckets=32)
+        got = run_generic(ta, mask, q, k, v, kv, B, heads, n_q, n_k, 0.125, **extra, **ropes)
+        for b, h in ((0, 0), (B // 2, 1), (B - 1, heads - 1)):
+            sel = slice(h * 64, h * 64 + 64)
+            qh, kh = q[b, :, sel], k[b, :, sel]
+            if ropes:
+                p0 = pos.get("q_pos0", 0)
+                qh = _ref.rope_f64(qh, ropes["rope_cos"][p0:], ropes["rope_sin"][p0:], n_q, 1)
+                kh = _ref.rope_f64(kh, ropes["rope_cos"], ropes["rope_sin"], n_k, 1)
+            allowed = _ref.allowed_matrix(mask, n_q, n_k, kv[b], **pos)
+            want = _ref.naive_attend(qh, kh, v[b, :, sel], allowed, 0.125, None if bias is None else bias[h])
+            assert _ref.scaled_err(got[b, :, sel], want) <= TOL, (B, b, h)

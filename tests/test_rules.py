@@ -1,0 +1,72 @@
+"""The choices of kernel, tile and split (csrc/rules.hpp) on both sides of their lines, on the CPU: the header is
+plain C++ and is compiled into a small program here."""
+import pathlib
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = pathlib.Path(__file__).resolve().parents[1] / "tsfm-zig_amd" / "csrc"
+CUS = 256
+
+MAIN = r"""
+#include <cstdio>
+#include <cstring>
+#include "rules.hpp"
+using namespace tsfm::rules;
+int main() {
+    char what[32];
+    while (scanf("%31s", what) == 1) {
+        if (!strcmp(what, "attn")) {
+            long rows; int n_q, n_k, mask, dense, rel, rope;
+            if (scanf("%ld %d %d %d %d %d %d", &rows, &n_q, &n_k, &mask, &dense, &rel, &rope) != 7) return 1;
+            AttnForm f = {rows, n_q, n_k, mask == 2 || mask == 3, mask == 5, mask == 4, mask == 1, dense != 0,
+                          rel != 0, rope != 0};
+            printf("%d\n", (int)attn_x3_pays(f, 256));
+        }
+    }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("clang++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    d = tmp_path_factory.mktemp("rules")
+    (d / "main.cpp").write_text(MAIN)
+    subprocess.run([cxx, "-std=c++17", "-Wall", "-Werror", "-I", str(CSRC), str(d / "main.cpp"), "-o", str(d / "main")],
+                   check=True)
+
+    def ask(*words):
+        out = subprocess.run([str(d / "main")], input=" ".join(str(w) for w in words), capture_output=True, text=True,
+                             check=True).stdout
+        return [int(x) for x in out.split()]
+
+    return ask
+
+
+FORMS = dict(plain=(0, 0, 0), dense=(1, 0, 0), t5=(0, 1, 0), rope=(0, 0, 1))
+FULL, KEYS_ADDITIVE, CAUSAL, CAUSAL_KEYS, FULL_KEYS, DECODER = range(6)
+
+
+@pytest.mark.parametrize("rows,n_q,mask,form,x3", [
+    # one row per CU or fewer: only where the bf16x3 kernel measured faster, form by form
+    (12, 64, KEYS_ADDITIVE, "rope", 0), (12, 66, KEYS_ADDITIVE, "rope", 1), (252, 109, FULL, "rope", 1),
+    (12, 66, KEYS_ADDITIVE, "plain", 0), (12, 69, KEYS_ADDITIVE, "plain", 1), (252, 66, FULL, "t5", 0),
+    (252, 128, KEYS_ADDITIVE, "t5", 1), (12, 129, KEYS_ADDITIVE, "t5", 0),
+    (12, 80, KEYS_ADDITIVE, "dense", 0), (252, 144, KEYS_ADDITIVE, "dense", 0), (252, 128, FULL, "dense", 0),
+    (252, 80, FULL_KEYS, "rope", 0), (12, 66, FULL_KEYS, "plain", 0), (12, 144, FULL_KEYS, "plain", 1),
+    (252, 144, FULL_KEYS, "rope", 0), (12, 72, DECODER, "rope", 0), (12, 72, DECODER, "plain", 1),
+    # more
+    (264, 37, KEYS_ADDITIVE, "rope", 1), (264, 7, KEYS_ADDITIVE, "rope", 0), (264, 33, KEYS_ADDITIVE, "rope", 0),
+    (768, 129, KEYS_ADDITIVE, "t5", 1), (264, 129, KEYS_ADDITIVE, "dense", 0), (516, 129, KEYS_ADDITIVE, "dense", 1),
+    (504, 144, KEYS_ADDITIVE, "dense", 0), (264, 144, KEYS_ADDITIVE, "dense", 1),
+    (768, 37, FULL_KEYS, "rope", 0), (264, 24, FULL_KEYS, "rope", 1), (504, 72, FULL_KEYS, "plain", 0),
+    (384, 72, FULL_KEYS, "plain", 1), (264, 16, KEYS_ADDITIVE, "plain", 0), (516, 16, KEYS_ADDITIVE, "plain", 1),
+    (384, 37, FULL, "plain", 0), (384, 37, KEYS_ADDITIVE, "plain", 1), (264, 32, DECODER, "rope", 1),
+    # the causal masks
+    (264, 109, CAUSAL, "rope", 0), (516, 95, CAUSAL_KEYS, "rope", 0), (516, 96, CAUSAL, "rope", 1)])
+def test_short_row_attention_kernel(rules, rows, n_q, mask, form, x3):
+    assert rules("attn", rows, n_q, 94 if mask == DECODER else n_q, mask, *FORMS[form]) == [x3]

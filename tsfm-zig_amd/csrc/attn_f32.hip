@@ -31,6 +31,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
+#include "rules.hpp"
 
 namespace tsfm {
 namespace {
@@ -751,29 +752,15 @@ hipError_t launch_bias(const Params& p, int bias, bool rope, hipStream_t s) {
 
 }  // namespace
 
-// Whether a call whose rows fit the resident kernel runs faster on the bf16x3 kernel (attn_x3.hip).
-// Launch times in us, resident / bf16x3, head count 12 (a key-masked call with RoPE unless said):
-//  - One row per CU or fewer: the resident kernel's 9 waves x 16 queries finish a row sooner up to 64
-//    queries (37: 7.4 / 8.3, 64: 8.4 / 8.5); past that the f32 instruction's rate shows (80: 11.6 / 10.5,
-//    109: 14.8 / 12.9, 144: 21.8 / 15.2). Rows of 32k + 1 queries, for which the bf16x3 kernel runs the
-//    last query on the VALU, stay resident (65: 9.3 / 14.0, 129: 16.7 / 19.8).
-//  - More rows than CUs: the resident kernel holds one per CU and takes them in rounds; the bf16x3
-//    kernel has three workgroups a CU in flight (264 rows: 37: 12.6 / 10.9, 109: 27.8 / 19.5, 129: 32.6 /
-//    28.0; decoder rows of 32 queries over 94 keys: 16.0 / 10.8, of 8 over 24: 8.1 / 6.0). Not for
-//    33 and 65 queries (11.8 / 12.8, 16.8 / 18.4) nor a handful of queries (one over 129 keys: 11.6 /
-//    13.1).
-//  - The causal masks: the resident kernel skips half its tiles and the two are even (94: 19.4 / 19.7 at
-//    384 rows, 12 rows 10.0 / 13.1) up to two rows per CU of at least 96 queries.
-static bool x3_pays(const Params& p, int mask) {
-    const int64_t rows = (int64_t)p.B * p.H, cus = device_cus();
-    const bool lone = p.n_q % 32 == 1;
-    if (mask == CAUSAL || mask == CAUSAL_KEYS) return p.n_q >= 96 && rows >= 2 * cus;
-    if (rows > cus) return p.n_q >= 8 && (!lone || p.n_q > 65);
-    return p.n_q > 64 && !lone;
+// Whether a call whose rows fit the resident kernel runs on the bf16x3 one (attn_x3.hip).
+static bool x3_pays(const Params& p, int mask, int bias, bool rope) {
+    const rules::AttnForm f = {(int64_t)p.B * p.H,  p.n_q, p.n_k, mask == CAUSAL || mask == CAUSAL_KEYS, mask == DECODER,
+                               mask == FULL_KEYS, mask == KEYS_ADDITIVE, bias == BIAS_DENSE, bias == BIAS_REL, rope};
+    return rules::attn_x3_pays(f, device_cus());
 }
 
 hipError_t launch_attn_f32(const Params& p, int mask, int bias, bool rope, hipStream_t s) {
-    if (p.n_k > kResidentKeys || x3_pays(p, mask)) return launch_attn_x3(p, mask, bias, rope, s);
+    if (p.n_k > kResidentKeys || x3_pays(p, mask, bias, rope)) return launch_attn_x3(p, mask, bias, rope, s);
     switch (mask) {
     case FULL: return launch_bias<FULL>(p, bias, rope, s);
     case KEYS_ADDITIVE: return launch_bias<KEYS_ADDITIVE>(p, bias, rope, s);

@@ -1,0 +1,70 @@
+// Which kernel, tile or split a call takes, from its sizes and form alone: host code without the GPU
+// runtime, so that the lines can be tested on any machine. cus: compute units of the device.
+#pragma once
+
+#include <stdint.h>
+
+namespace tsfm {
+namespace rules {
+
+// Whether f32 attention whose rows fit the kernel with resident keys (attn_f32.hip) runs faster on the bf16x3
+// kernel (attn_x3.hip). Launch times in us, resident / bf16x3, at 12 heads; "rows" are (series, head) pairs.
+// A row of 32k + 1 queries (lone) costs the bf16x3 kernel a pass of its own for the last one.
+struct AttnForm {
+    int64_t rows;
+    int n_q, n_k;
+    bool causal;     // CAUSAL, CAUSAL_KEYS
+    bool decoder;    // DECODER
+    bool keys_hard;  // FULL_KEYS: invalid keys at -inf, so every chunk with one goes through the mask rule
+    bool keys_soft;  // KEYS_ADDITIVE (neither of the four: FULL)
+    bool dense;      // a dense bias, read per score in either kernel
+    bool rel;        // the T5 table
+    bool rope;
+};
+inline bool attn_x3_pays(const AttnForm& f, int64_t cus) {
+    const bool lone = f.n_q % 32 == 1;
+    // The causal masks: the resident kernel skips half its tiles. Past two rows per CU and 96 queries the
+    // bf16x3 kernel wins (516 rows of 96 queries: 29.4 / 20.9).
+    const bool many = f.rows >= 2 * cus && f.n_q >= 96;
+    if (f.causal) return many;
+    if (f.rows <= cus) {
+        // One row per CU or fewer: the resident kernel's nine waves of 16 queries finish a row sooner up to 64
+        // queries (12 rows with RoPE, key-masked: 64: 8.4 / 8.6, 66: 11.2 / 10.3, 109: 14.8 / 12.9), and
+        // without RoPE, where it stages by DMA, up to 68 (plain 66: 9.3 / 9.7, 69: 10.4 / 10.0; T5 66: 9.4 /
+        // 10.1 with all keys valid). Scores that need work of their own there cost the bf16x3 kernel more:
+        // a dense bias (128: 16.3 / 19.5, 252 rows of 144: 25.4 / 34.8), hard key masks (80 with RoPE:
+        // 11.8 / 14.0, plain 66: 9.4 / 12.1; from 130 on it wins while two workgroups a row fit the
+        // CUs, 144: 22.6 / 19.8) and decoder rows with RoPE (72 over 144: 1.04).
+        if (lone || f.dense || (f.decoder && f.rope)) return false;
+        if (f.keys_hard) return !f.rel && f.n_q > 128 && 2 * f.rows <= cus;
+        return f.n_q > (f.rope ? 64 : 68);
+    }
+    // More rows than CUs: the resident kernel holds one per CU and takes them in rounds; the bf16x3 kernel has
+    // three workgroups a CU in flight (264 rows, key-masked with RoPE: 37: 12.6 / 10.9, 109: 27.8 / 19.5; decoder
+    // rows of 32 queries over 94 keys: 16.0 / 10.8). Not for a handful of queries (one over 129 keys: 11.6 /
+    // 13.1), nor 33 and 65 (11.8 / 12.8, 16.8 / 18.4).
+    if (f.n_q < 8) return false;
+    const bool heavy = f.dense || f.keys_hard || (f.decoder && f.rope);
+    if (lone) return f.n_q > 65 && (many || !heavy);
+    // Just under a whole number of rows per CU the resident kernel's last round is full: heavy scores lose there
+    // (504 rows of 144, dense: 1.30, hard masks 1.1-1.23; of 72, hard masks: 1.08), except from 96 to 128
+    // queries.
+    const bool slack = f.rows % cus <= cus * 3 / 4;
+    if (f.keys_hard) {
+        // 8-16: 6.5 / 7.4, 17-32: 0.82-1.0, 33-64: 10.7 / 11.7 at 264 rows and 1.25 at 768.
+        if (f.n_q <= 16 || (f.n_q > 32 && f.n_q <= 64)) return false;
+        if (f.n_q >= 96 && f.dense) return many;
+        return slack || (f.n_q >= 96 && f.n_q <= 128) || many;
+    }
+    if (f.dense) return slack || f.n_q <= 128 || many;
+    if (!f.rope && !f.decoder && f.rows < 2 * cus && f.n_k <= 64) {
+        // Short rows by DMA: 34 queries (1.06; with all keys valid 1.13, and up to 48 1.0-1.04), and, without
+        // the T5 table either, up to 16 (6.3 / 6.6, 6.4 / 7.0).
+        if (f.n_q > 32 && f.n_q <= (f.keys_soft || f.rel ? 34 : 48)) return false;
+        if (!f.rel && f.n_q <= 16 && f.n_k <= 16) return false;
+    }
+    return true;
+}
+
+}  // namespace rules
+}  // namespace tsfm
