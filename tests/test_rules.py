@@ -7,7 +7,6 @@ import subprocess
 import pytest
 
 CSRC = pathlib.Path(__file__).resolve().parents[1] / "tsfm-zig_amd" / "csrc"
-CUS = 256
 
 MAIN = r"""
 #include <cstdio>
@@ -23,6 +22,10 @@ int main() {
             AttnForm f = {rows, n_q, n_k, mask == 2 || mask == 3, mask == 5, mask == 4, mask == 1, dense != 0,
                           rel != 0, rope != 0};
             printf("%d\n", (int)attn_x3_pays(f, 256));
+        } else if (!strcmp(what, "big")) {
+            long d_in, cus; int pre;
+            if (scanf("%ld %d %ld", &d_in, &pre, &cus) != 3) return 1;
+            printf("%d\n", (int)big_tiles_min(d_in, pre != 0, cus));
         }
     }
 }
@@ -70,3 +73,12 @@ FULL, KEYS_ADDITIVE, CAUSAL, CAUSAL_KEYS, FULL_KEYS, DECODER = range(6)
     (264, 109, CAUSAL, "rope", 0), (516, 95, CAUSAL_KEYS, "rope", 0), (516, 96, CAUSAL, "rope", 1)])
 def test_short_row_attention_kernel(rules, rows, n_q, mask, form, x3):
     assert rules("attn", rows, n_q, 94 if mask == DECODER else n_q, mask, *FORMS[form]) == [x3]
+
+
+@pytest.mark.parametrize("d_in,presplit,cus,tiles", [
+    (768, 0, 256, 200), (512, 0, 256, 200), (768, 1, 256, 160), (512, 1, 256, 200), (1024, 1, 128, 80),
+    (48, 0, 256, 256), (176, 0, 256, 256), (528, 0, 256, 200), (48, 0, 128, 128)])
+def test_tiles_from_which_a_product_runs_on_the_big_ones(rules, d_in, presplit, cus, tiles):
+    """The reductions that run on the f32 instruction (not of whole 32s) keep a full round of the small tiles, four a
+    CU: 1100 to 1200 rows of the Chronos-2 patch embedding (48 values, 3072 columns) are 216 and 240 big tiles."""
+    assert rules("big", d_in, presplit, cus) == [tiles]

@@ -756,7 +756,8 @@ hipError_t launch_bias(const Params& p, int bias, bool rope, hipStream_t s) {
 static bool x3_pays(const Params& p, int mask, int bias, bool rope) {
     const rules::AttnForm f = {(int64_t)p.B * p.H,  p.n_q, p.n_k, mask == CAUSAL || mask == CAUSAL_KEYS, mask == DECODER,
                                mask == FULL_KEYS, mask == KEYS_ADDITIVE, bias == BIAS_DENSE, bias == BIAS_REL, rope};
-    return rules::attn_x3_pays(f, device_cus());
+    const int cus = device_cus();
+    return cus > 0 && rules::attn_x3_pays(f, cus);  // (0: no device, refused by the launch)
 }
 
 hipError_t launch_attn_f32(const Params& p, int mask, int bias, bool rope, hipStream_t s) {

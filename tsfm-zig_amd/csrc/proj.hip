@@ -37,6 +37,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
+#include "rules.hpp"
 
 namespace tsfm {
 namespace {
@@ -1094,17 +1095,10 @@ hipError_t launch_weight_planes(const float* w, int64_t w_ld, int rows, int cols
 
 namespace {
 
-// The unsplit product. BIG tiles when there are enough of them for every CU; SMALL ones take
+// The unsplit product, on BIG or SMALL tiles (rules::big_tiles_min); SMALL ones take
 // 32-wide steps when d_in allows (half the step barriers), else 16-wide. The accumulation chunks
 // are the same units of 16 p.chunk indices either way, so the result depends on neither the step
 // width nor the tile shape, and one product may mix the two.
-// A SMALL tile is a quarter of a BIG one, and the SMALL kernels hold three workgroups a CU (the split
-// inside the product) or two (pre-split operands), the BIG ones one. So BIG tiles pay from where the
-// SMALL ones would start another round, not from a tile for every CU: above 192 of 256 CUs, and (with
-// some room) 128. Measured (us, SMALL / BIG): the Chronos-2 q/k/v product of 1500 rows (216 tiles)
-// 54 / 44, of 1200 (180) 40 / 43; pre-split, the Chronos-2 layers of 4820 rows 1505 / 1432 and the
-// Chronos-Bolt forecast of 32 x 2048 steps 1681 / 1577 (198 tiles of 4128 rows).
-constexpr int64_t kBigTilesMin = 200, kBigTilesMinPre = 160;
 template <int OUT>
 hipError_t launch_small(ProjParams p, hipStream_t stream) {
     p.m_tiles = (p.tokens - p.m_base + BM - 1) / BM;
@@ -1132,7 +1126,9 @@ hipError_t launch_unsplit(ProjParams p, hipStream_t stream) {
     // The token rows from p.m_base on (0 at the first call).
     const int64_t rows = (int64_t)p.tokens - p.m_base;
     const int64_t big_m = (rows + 127) / 128, big_n = (p.width * p.n_out + 127) / 128;
-    if (big_m * big_n < (p.xp != nullptr ? kBigTilesMinPre : kBigTilesMin)) return launch_small<OUT>(p, stream);
+    // (A handful of tiles is few for any device: no need to ask for its CUs.)
+    if (big_m * big_n < 64 || big_m * big_n < rules::big_tiles_min(p.d_in, p.xp != nullptr, device_cus()))
+        return launch_small<OUT>(p, stream);
     if (p.d_in % X3_BK == 0 && p.xp != nullptr && p.splits <= 1 && p.m_base == 0) {
         // Pre-split operands: 256 x 128 tiles, one workgroup per CU, in whole rounds; the token rows
         // past them go to 128 x 128 / 64 x 64 tiles below.

@@ -66,5 +66,23 @@ inline bool attn_x3_pays(const AttnForm& f, int64_t cus) {
     return true;
 }
 
+// Tiles of 128 x 128 from which a product runs on them (BIG), and on 64 x 64 ones (SMALL, a quarter of the
+// work) below. BIG tiles pay from where the SMALL ones would start another round, not from a tile for every
+// CU. Launch times in us, SMALL / BIG, at 256 CUs:
+//  - Split inside the product: three SMALL workgroups a CU, one BIG: past 192 tiles (768 indices: 180 tiles 41.5 /
+//    41.8, 198 56.1 / 42.5, 216 56.1 / 43.8).
+//  - Pre-split operands: two SMALL workgroups a CU, so past 128, with room for the sharing that SMALL tiles lose
+//    late (1024 indices, 2048 columns: 162 tiles of 768 indices 49.6 / 46.3; Chronos-2 layers of 4820 rows 1505 /
+//    1432). Short reductions keep SMALL ones up to a round of the others (512 indices, 162 tiles 37.6 / 38.5,
+//    192 38.2 / 39.5, 216 43.1 / 39.9).
+//  - The f32 instruction (reductions not of whole 32s): four SMALL workgroups a CU, two BIG, so a round of SMALL
+//    ones lasts to 256 tiles; from 512 indices on BIG ones read their operands less often (528: 204 tiles
+//    45.4 / 42.9, 1040: 216 82.8 / 76.6; 176: 19.6 / 19.7, with RoPE 20.7 / 21.5; 48: 9.9 / 11.0).
+inline int64_t big_tiles_min(int64_t d_in, bool presplit, int64_t cus) {
+    const int64_t thin = cus * 25 / 32, round = cus;  // 200 and 256 tiles
+    if (d_in % 32 != 0) return d_in >= 512 ? thin : round;
+    return presplit && d_in >= 768 ? cus * 5 / 8 : thin;  // (160 tiles)
+}
+
 }  // namespace rules
 }  // namespace tsfm
