@@ -374,11 +374,13 @@ def test_presplit_product_back_to_back_launches_agree(ta, gpu_ready):
 
 
 @pytest.mark.parametrize("b,seq,d,nh", [(12, 125, 768, 12), (20, 130, 512, 5), (20, 126, 512, 5), (16, 128, 512, 6),
-                                        (3, 1365, 768, 4), (9, 125, 48, 16), (20, 105, 528, 8), (18, 128, 1024, 7)])
+                                        (3, 1365, 768, 4), (9, 125, 48, 16), (20, 105, 528, 8), (18, 128, 1024, 7),
+                                        (2, 101, 4096, 8), (4, 150, 2048, 8), (5, 153, 1536, 8), (9, 148, 1024, 16)])
 def test_tile_choice_between_the_kernels(ta, gpu_ready, b, seq, d, nh):
     """Products around the rules of tile and operand form: 216 tiles of 128 x 128 split inside the
     product, 168 and 160 on pre-split operands over 2600 and 2520 rows, 2048 and 4095 rows of at
-    least 2^30 multiply-adds, 216 and 204 tiles of the f32 instruction and 198 of longer pre-split rows: tsfm_qkv_project (operand workspace) and tsfm_qkv_project_noalloc (none)
+    least 2^30 multiply-adds, 216 and 204 tiles of the f32 instruction, 198 of longer pre-split rows,
+    and fewer rows of long reductions or of much work: tsfm_qkv_project (operand workspace) and tsfm_qkv_project_noalloc (none)
     give the same bits, within the bar of float64."""
     import torch
 

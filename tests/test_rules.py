@@ -22,6 +22,10 @@ int main() {
             AttnForm f = {rows, n_q, n_k, mask == 2 || mask == 3, mask == 5, mask == 4, mask == 1, dense != 0,
                           rel != 0, rope != 0};
             printf("%d\n", (int)attn_x3_pays(f, 256));
+        } else if (!strcmp(what, "planes")) {
+            long tokens, d_in, cols; int whole;
+            if (scanf("%ld %ld %ld %d", &tokens, &d_in, &cols, &whole) != 4) return 1;
+            printf("%d\n", (int)planes_pay(tokens, d_in, cols, whole != 0, 256));
         } else if (!strcmp(what, "big")) {
             long d_in, cus; int pre;
             if (scanf("%ld %d %ld", &d_in, &pre, &cus) != 3) return 1;
@@ -82,3 +86,17 @@ def test_tiles_from_which_a_product_runs_on_the_big_ones(rules, d_in, presplit, 
     """The reductions that run on the f32 instruction (not of whole 32s) keep a full round of the small tiles, four a
     CU: 1100 to 1200 rows of the Chronos-2 patch embedding (48 values, 3072 columns) are 216 and 240 big tiles."""
     assert rules("big", d_in, presplit, cus) == [tiles]
+
+
+@pytest.mark.parametrize("tokens,d_in,cols,whole,pre", [
+    # long reductions that cannot be shared out: q/k/v products with RoPE
+    (200, 4096, 1536, 1, 1), (768, 4096, 1536, 1, 1), (484, 3072, 2304, 1, 1), (545, 2048, 1536, 1, 1),
+    (768, 1536, 1536, 1, 1), (545, 1536, 1536, 1, 0), (128, 2048, 6144, 1, 0), (64, 4096, 1536, 1, 0),
+    (768, 768, 2304, 1, 0), (1928, 768, 2304, 1, 0), (1500, 1536, 1536, 1, 0),
+    # the same without RoPE: shared out, or tiles enough
+    (200, 4096, 1536, 0, 0), (545, 2048, 1536, 0, 0), (1205, 2048, 1536, 0, 1), (400, 2048, 6144, 0, 0),
+    # by work and rows
+    (1332, 1024, 3072, 1, 1), (1205, 1024, 3072, 0, 0), (999, 1024, 4096, 0, 0), (1332, 1024, 4096, 0, 1),
+    (1500, 3072, 768, 0, 0), (2048, 768, 768, 0, 1), (2048, 512, 512, 0, 0), (2600, 1040, 2304, 0, 0)])
+def test_presplit_operands(rules, tokens, d_in, cols, whole, pre):
+    assert rules("planes", tokens, d_in, cols, whole) == [pre]

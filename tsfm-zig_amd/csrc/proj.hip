@@ -1039,18 +1039,14 @@ size_t plane_operand_bytes(int64_t rows, int64_t cols) {
     if (rows <= 0 || cols <= 0 || cols % X3_BK) return 0;
     return (size_t)((rows + 15) / 16) * (size_t)(cols / X3_BK) * 3 * kPlaneChunk;
 }
-// Products that run on pre-split operands when a workspace is lent: at least 2^30 multiply-adds over
-// at least 2048 rows, or 5 2^30 over fewer. Splitting the weights costs the same at any row count
-// and saves each row tile its own split, so it pays by rows (whole calls in us, pre-split / split
-// inside the product: Chronos-2 layers of 484 rows 500 / 457, 1205 rows 675 / 634, 1928 rows 886 / 867,
-// 4820 rows 1513 / 1707; Timestral q/k/v/gate, 4096 columns: 333 rows 43 / 39, 999 rows 62 / 57, 1332
-// rows 87 / 93).
-static bool planes_pay(int64_t tokens, int64_t d_in, int64_t n_cols) {
-    const int64_t macs = tokens * n_cols * d_in, unit = (int64_t)1 << 30;
-    return d_in % X3_BK == 0 && macs >= unit && (tokens >= 2048 || macs >= 5 * unit);
+// whole: as rules::planes_pay (a caller that splits the product's input ahead may pass false: the
+// narrower answer).
+static bool planes_pay(int64_t tokens, int64_t d_in, int64_t n_cols, bool whole) {
+    // (Asking for the device's CUs takes 0.3 us of the host: not for the small products, which never do.)
+    return tokens * n_cols * d_in >= (int64_t)1 << 30 && rules::planes_pay(tokens, d_in, n_cols, whole, device_cus());
 }
 bool proj_planes_ready(int64_t tokens, int64_t d_in, int64_t n_cols) {
-    return t_plane_ws != nullptr && planes_pay(tokens, d_in, n_cols) &&
+    return t_plane_ws != nullptr && planes_pay(tokens, d_in, n_cols, false) &&
            plane_operand_bytes(n_cols, d_in) <= t_plane_bytes;
 }
 hipError_t launch_rms_norm_planes(const float* x, int64_t x_tok, void* planes, const float* scale, int rows, int dim,
@@ -1208,7 +1204,7 @@ bool proj_fuses_input_norm(int64_t tokens, int64_t d_in) {
     return tokens > 0 && tokens <= kSkinnyTokens && d_in > 0 && d_in <= kSkinnyNormIn && d_in % 16 == 0;
 }
 
-constexpr int64_t kSplitBlocks = 420;
+using rules::kSplitBlocks;
 size_t proj_split_bytes(ProjParams& p) {
     p.m_tiles = (p.tokens + BM - 1) / BM;
     p.n_tiles = (p.width * p.n_out + BN - 1) / BN;
@@ -1279,7 +1275,8 @@ hipError_t launch_proj(const ProjParams& p0, hipStream_t stream) {
     if (((p.x_pre != nullptr || p.y_planes != nullptr || p.w_pre != nullptr) && !ready) ||
         (p.y_planes != nullptr && (p.n_out != 1 || p.width % X3_BK || p.out_dtype != 0 || p.rope_cos != nullptr)))
         return hipErrorInvalidValue;
-    if (p.w_pre != nullptr || (t_plane_ws != nullptr && planes_pay(p.tokens, p.d_in, n_cols))) {
+    const bool whole = p.rope_cos != nullptr || p.out_dtype != 0;
+    if (p.w_pre != nullptr || (t_plane_ws != nullptr && planes_pay(p.tokens, p.d_in, n_cols, whole))) {
         const size_t xb = p.x_pre != nullptr ? 0 : plane_operand_bytes(p.tokens, p.d_in);
         const size_t wb = p.w_pre != nullptr ? 0 : plane_operand_bytes(n_cols, p.d_in);
         if (xb + wb <= (t_plane_ws != nullptr ? t_plane_bytes : 0)) {

@@ -84,5 +84,34 @@ inline int64_t big_tiles_min(int64_t d_in, bool presplit, int64_t cus) {
     return presplit && d_in >= 768 ? cus * 5 / 8 : thin;  // (160 tiles)
 }
 
+// Tiles of 64 x 64 from which a product never shares its reduction out over workgroups (proj_split_bytes).
+constexpr int64_t kSplitBlocks = 420;
+
+// Whether a product runs on pre-split operands when a workspace is lent, instead of splitting inside. Splitting
+// the weights costs the same at any row count and saves each row tile its own split, so it pays by rows and by
+// the work of the product. Pre-split / split inside, over some 1300 products of 64 to 2600 rows and 512 to 4096
+// indices (whole calls in us: Chronos-2 layers of 484 rows 500 / 457, 1205 rows 675 / 634, 4820 rows 1513 /
+// 1707; Timestral q/k/v/gate, 4096 columns: 999 rows 62 / 57, 1332 rows 87 / 93):
+//  - From 2048 rows or 5 2^30 multiply-adds on: 0.83-1.0 (reductions of 512 up to 1.3).
+//  - With less work, a product that shares its reduction out loses (200 rows of 4096 indices, 1536 columns: 1.19).
+//    One that cannot (whole: RoPE, half-precision outputs; or tiles enough without) walks all of it in each
+//    tile, and its own split with it. There pre-split wins for long reductions at any size (4096 indices, 1536
+//    columns: 200 rows 81 / 97, 768 rows 99 / 124; 1536 from 1.5 2^30 on: 900 rows 0.92), for others at 4.5
+//    2^30, at 1200 rows and more 3.75 2^30 (1024 indices, 3072 columns: 1205 rows 1.02, 1332 0.95, 1500 80 /
+//    84). Not for more than 4096 columns, whose weights take longer to split (2048 indices, 6144 columns: 128
+//    rows 1.13), nor where its tiles, two a CU, start a second round that three a CU do not (1500 rows of
+//    1536 indices, 1536 columns: 77 / 69).
+// whole: the product's form keeps it from sharing its reduction out.
+inline bool planes_pay(int64_t tokens, int64_t d_in, int64_t n_cols, bool whole, int64_t cus) {
+    const int64_t macs = tokens * n_cols * d_in, quarter = (int64_t)1 << 28;  // (quarters of 2^30)
+    if (d_in % 32 != 0 || macs < 4 * quarter) return false;
+    if (tokens >= 2048 || macs >= 20 * quarter) return true;
+    const int64_t blocks = (tokens + 63) / 64 * ((n_cols + 63) / 64);
+    if ((!whole && blocks < kSplitBlocks) || n_cols > 4096) return false;
+    if (blocks > 2 * cus && blocks < 4 * big_tiles_min(d_in, true, cus)) return false;
+    if (d_in >= 2048 || (d_in >= 1536 && macs >= 6 * quarter)) return true;
+    return macs >= (tokens < 1200 ? 18 : 15) * quarter;
+}
+
 }  // namespace rules
 }  // namespace tsfm
