@@ -26,6 +26,22 @@ int main() {
             long tokens, d_in, cols; int whole;
             if (scanf("%ld %ld %ld %d", &tokens, &d_in, &cols, &whole) != 4) return 1;
             printf("%d\n", (int)planes_pay(tokens, d_in, cols, whole != 0, 256));
+        } else if (!strcmp(what, "split")) {
+            long tokens, d_in, cols;
+            if (scanf("%ld %ld %ld", &tokens, &d_in, &cols) != 3) return 1;
+            const Split s = reduction_split((tokens + 63) / 64 * ((cols + 63) / 64), (int)(d_in / 16), d_in % 32 == 0,
+                                            [] { return 256; });
+            printf("%d %d\n", s.shares, s.steps);
+        } else if (!strcmp(what, "splits")) {  // the most shares of 64 x 64 tiles any product has
+            long most = 0;
+            for (long blocks = 1; blocks < 2000; blocks++)
+                for (int steps = 1; steps <= 512; steps++)
+                    for (int pairs = 0; pairs < 2; pairs++) {
+                        const Split s = reduction_split(blocks, steps, pairs != 0, [] { return 256; });
+                        if (s.shares < 1 || s.steps * s.shares < steps || s.steps * (s.shares - 1) >= steps) return 2;
+                        if (s.shares > 1 && s.shares * blocks > most) most = s.shares * blocks;
+                    }
+            printf("%ld\n", most);
         } else if (!strcmp(what, "big")) {
             long d_in, cus; int pre;
             if (scanf("%ld %d %ld", &d_in, &pre, &cus) != 3) return 1;
@@ -100,3 +116,19 @@ def test_tiles_from_which_a_product_runs_on_the_big_ones(rules, d_in, presplit, 
     (1500, 3072, 768, 0, 0), (2048, 768, 768, 0, 1), (2048, 512, 512, 0, 0), (2600, 1040, 2304, 0, 0)])
 def test_presplit_operands(rules, tokens, d_in, cols, whole, pre):
     assert rules("planes", tokens, d_in, cols, whole) == [pre]
+
+
+@pytest.mark.parametrize("tokens,d_in,cols,shares", [
+    (33, 2048, 4096, 8), (8, 4096, 2048, 16), (17, 1024, 4096, 8),  # 512 workgroups, two a CU
+    (545, 768, 768, 4), (528, 512, 1536, 2), (545, 768, 2304, 2),  # about 420
+    (448, 256, 3 * 24 * 64, 1), (64, 256, 3 * 139 * 64, 2), (64, 256, 3 * 140 * 64, 1), (64, 240, 512, 1)])
+def test_shares_of_a_reduction(rules, tokens, d_in, cols, shares):
+    got, steps = rules("split", tokens, d_in, cols)
+    assert got == shares and steps * got >= d_in // 16
+
+
+def test_shares_cover_the_reduction_and_fit_the_fixed_array(rules):
+    """Every share has steps to walk, and the partial sums of no product pass the 16 MiB array of
+    tsfm_qkv_project_noalloc: at most 2 x 419 tiles of 64 x 64 floats, the figure in its header."""
+    most = rules("splits")[0]
+    assert most == 2 * 419 and most * 64 * 64 * 4 == 13729792 <= 16 << 20

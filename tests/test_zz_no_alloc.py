@@ -96,19 +96,30 @@ def test_noalloc_refuses_host_pointers(ta, gpu_ready):
     assert lib.tsfm_qkv_project_noalloc(ctypes.byref(a)) == ta.E_UNSUPPORTED
 
 
-def test_noalloc_holds_the_largest_split_partials(ta, gpu_ready):
-    """The split rule aims at about 512 workgroups: a product of b < 512 tiles of 64 x 64 splits
-    ceil(512 / b) ways at most, so its partials never exceed 2 x 511 tiles (16.7 MB, under the
-    array's 16 MiB). 448 tokens x 3 x 24 heads = 7 x 72 = 504 tiles, two splits over d_in 256:
-    16.5 MB of partials, the same bits as tsfm_qkv_project."""
+def _unsplit(torch, ta, c):
+    """q, k and v as a product of this case gives them when it runs unsplit: with RoPE tables of angle 0."""
+    x, ws, _, tokens, d, nh = c
+    one, zero = torch.ones(tokens, 32, device="cuda"), torch.zeros(tokens, 32, device="cuda")
+    return _run(torch, ta, ta.load().tsfm_qkv_project, (x, ws, (one, zero), tokens, d, nh))
+
+
+@pytest.mark.parametrize("tokens,nh", [(64, 139), (448, 19)])
+def test_noalloc_holds_the_largest_split_partials(ta, gpu_ready, tokens, nh):
+    """A product splits its reduction up to 419 tiles of 64 x 64, two ways there: 64 tokens x 3 x 139 heads = 417
+    tiles and 448 x 3 x 19 = 399, 13.7 and 13.1 MB of partials in the 16 MiB array. The same bits as
+    tsfm_qkv_project, and other bits than the same product unsplit: the partials were written and added."""
     import torch
 
     lib = _lib(ta)
-    c = _case(torch, 6, 448, 256, 24)
+    c = _case(torch, 6, tokens, 256, nh)
     want = _run(torch, ta, lib.tsfm_qkv_project, c)
     got = _run(torch, ta, lib.tsfm_qkv_project_noalloc, c)
     for g, w_ in zip(got, want):
         assert np.array_equal(g, w_)
+    whole = _unsplit(torch, ta, c)
+    assert any((g != w_).any() for g, w_ in zip(got, whole))
+    for g, w_ in zip(got, whole):
+        assert _ref.scaled_err(g, w_) <= 1e-5
 
 
 @pytest.mark.parametrize("tokens,nh", [(448, 19), (448, 20), (64, 139), (64, 140)])

@@ -1204,7 +1204,6 @@ bool proj_fuses_input_norm(int64_t tokens, int64_t d_in) {
     return tokens > 0 && tokens <= kSkinnyTokens && d_in > 0 && d_in <= kSkinnyNormIn && d_in % 16 == 0;
 }
 
-using rules::kSplitBlocks;
 size_t proj_split_bytes(ProjParams& p) {
     p.m_tiles = (p.tokens + BM - 1) / BM;
     p.n_tiles = (p.width * p.n_out + BN - 1) / BN;
@@ -1214,29 +1213,17 @@ size_t proj_split_bytes(ProjParams& p) {
     p.split_steps = steps;
     p.partial = nullptr;
     if (p.x_pre != nullptr || p.y_planes != nullptr || p.w_pre != nullptr) return 0;  // pre-split operands: never split
-    // f32 outputs, no RoPE; several outputs only without an epilogue; fewer tiles than kSplitBlocks,
-    // and at least 16 steps to share out.
-    if (!((p.n_out == 1 || p.epi == kEpiNone) && p.rope_cos == nullptr && p.out_dtype == 0 && blocks < kSplitBlocks &&
-          steps >= 16) ||
+    // f32 outputs, no RoPE; several outputs only without an epilogue.
+    if (!((p.n_out == 1 || p.epi == kEpiNone) && p.rope_cos == nullptr && p.out_dtype == 0 &&
+          blocks < rules::kSplitBlocks) ||
         skinny(p))
         return 0;
-    // About kSplitBlocks workgroups: each split costs its start, its partial sums' trip through memory and
-    // the longer sum afterwards (half of an 18 us launch of 576 workgroups), so a product splits only
-    // while the CUs have fewer than about one and a half workgroups each. Whole calls in us, aiming at
-    // 360 / 420 / 470 / 512 workgroups: Chronos-2 layers of 545 rows 434 / 432 / 454 / 466, the
-    // Chronos-Bolt-small forecast 971 / 936 / 940 / 948, Chronos-Bolt-base layers of 528 rows 467 / 464 /
-    // 490 / 492, of 1056 rows 706 / 693 / 691 / 693.
-    int s = (int)std::min<int64_t>((kSplitBlocks + blocks - 1) / blocks, std::min(steps / 8, 16));
-    if (s < 2) return 0;
-    int per = (steps + s - 1) / s;
-    if (p.d_in % X3_BK == 0) per += per & 1;  // whole 32-index steps for the bf16x3 kernel
-    s = (steps + per - 1) / per;
-    if (s < 2) return 0;
-    p.splits = s;
-    p.split_steps = per;
-    // s * blocks <= kSplitBlocks + blocks - 1 < 1536 and tokens * width <= blocks * BM * BN, so the partials
-    // always fit kSplitWorkspaceBytes.
-    return (size_t)s * p.tokens * p.width * p.n_out * sizeof(float);
+    const rules::Split sp = rules::reduction_split(blocks, steps, p.d_in % X3_BK == 0, device_cus);
+    if (sp.shares < 2) return 0;
+    p.splits = sp.shares;
+    p.split_steps = sp.steps;
+    // At most two shares of 419 tiles, so the partials always fit kSplitWorkspaceBytes.
+    return (size_t)sp.shares * p.tokens * p.width * p.n_out * sizeof(float);
 }
 
 hipError_t launch_proj(const ProjParams& p0, hipStream_t stream) {

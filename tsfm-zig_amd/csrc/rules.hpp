@@ -84,8 +84,43 @@ inline int64_t big_tiles_min(int64_t d_in, bool presplit, int64_t cus) {
     return presplit && d_in >= 768 ? cus * 5 / 8 : thin;  // (160 tiles)
 }
 
-// Tiles of 64 x 64 from which a product never shares its reduction out over workgroups (proj_split_bytes).
-constexpr int64_t kSplitBlocks = 420;
+// How many workgroups share a tile's reduction of `steps` 16-wide steps, and how many steps each takes, for a
+// product of `blocks` tiles of 64 x 64. pairs: shares of an even number of steps (32-wide ones).
+//
+// Each share costs its start, its partial sums' trip through memory and the longer sum afterwards (half of an
+// 18 us launch of 576 workgroups), so a product is shared out only while the CUs have fewer than about one and
+// a half workgroups each: aiming at 360 / 420 / 470 / 512 workgroups, Chronos-2 layers of 545 rows take 434 /
+// 432 / 454 / 466 us, the Chronos-Bolt-small forecast 971 / 936 / 940 / 948, Chronos-Bolt-base layers of 528
+// rows 467 / 464 / 490 / 492. Where 512 deals the CUs their workgroups evenly and 420 does not (32 or 64 tiles:
+// 16 or 8 shares against 13 or 7), the fullest CU has less to do with 512: four outputs of 2048 indices, 1024
+// columns each, 33 rows 18.8 / 17.1 us; 4096 indices, 512 columns, 8 rows 18.3 / 17.1.
+struct Split {
+    int shares, steps;  // shares: 1 = unsplit
+};
+constexpr int64_t kSplitBlocks = 420;  // tiles from which the reduction is never shared out
+inline Split split_aiming_at(int64_t workgroups, int64_t blocks, int steps, bool pairs) {
+    const Split whole = {1, steps};
+    if (steps < 16) return whole;
+    int64_t s = (workgroups + blocks - 1) / blocks;
+    if (s > steps / 8) s = steps / 8;
+    if (s > 16) s = 16;
+    if (s < 2) return whole;
+    int per = (int)((steps + s - 1) / s);
+    if (pairs) per += per & 1;
+    s = (steps + per - 1) / per;
+    return s < 2 ? whole : Split{(int)s, per};
+}
+// device_cus: asked only where the two differ (it takes 0.3 us of the host).
+template <class Cus>
+inline Split reduction_split(int64_t blocks, int steps, bool pairs, Cus&& device_cus) {
+    if (blocks <= 0 || blocks >= kSplitBlocks) return {1, steps};
+    const Split a = split_aiming_at(kSplitBlocks, blocks, steps, pairs), b = split_aiming_at(512, blocks, steps, pairs);
+    if (a.shares == b.shares) return a;
+    const int64_t cus = device_cus();
+    // Steps the fullest CU walks.
+    auto longest = [&](const Split& s) { return (s.shares * blocks + cus - 1) / cus * s.steps; };
+    return cus > 0 && longest(b) < longest(a) ? b : a;
+}
 
 // Whether a product runs on pre-split operands when a workspace is lent, instead of splitting inside. Splitting
 // the weights costs the same at any row count and saves each row tile its own split, so it pays by rows and by
