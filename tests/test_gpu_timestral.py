@@ -420,12 +420,11 @@ def test_timestral_rows_longer_than_a_tile(ta, orc, orc16, gpu_ready, length, ps
                                                              (32, 1, 96, False, True, True),
                                                              (13, 2, 128, True, False, True)])
 def test_timestral_weights_split_once_per_call(ta, orc, orc16, gpu_ready, b, v, hid, gated, kv_cache, use_asinh):
-    """Forecasts of several decode blocks with at least 2048 tokens in all: the layers' weights are split
-    once per call, the norms, gates and MLP activations written split for the products of the blocks
-    of at least 768 tokens (ragged row blocks, hidden widths of 3 to 5 chunks, with and without
-    gates), the shorter blocks splitting inside their products. Against both oracle builds and
-    float64; in bf16 against the f32 forecast."""
-    length, horizon, per_shot = 470, 80, 3
+    """Forecasts with two decode blocks of at least 768 tokens and 2048 together: the layers' weights are
+    split once per call, the norms, gates and MLP activations written split for the products (ragged row
+    blocks, hidden widths of 3 to 5 chunks, with and without gates); a last, shorter block splits inside
+    its products. Against both oracle builds and float64; in bf16 against the f32 forecast."""
+    length, horizon, per_shot = 470, 22 * 16 - 5, 10
     rng = np.random.default_rng(b + hid)
     m = _ref.timestral_model(rng, d=128, nh=2, hid=hid, schedule=("time_variate", "time"), use_asinh=use_asinh,
                              gated=gated)
@@ -433,8 +432,9 @@ def test_timestral_weights_split_once_per_call(ta, orc, orc16, gpu_ready, b, v, 
     x = (20 + 6 * np.sin(2 * np.pi * t / 24) + 0.02 * t + rng.standard_normal((b * v, length))).astype(np.float32)
     obs = rng.random((b * v, length)) >= 0.1
     x[~obs] = 0
-    rows = 2 * b * v  # blocks of 3 and 2 patches after 30 of context
-    assert rows * (30 + 3) >= 768 and rows * (30 + 3 + (3 if kv_cache else 33) + 2) >= 2048
+    rows = 2 * b * v  # blocks of 10, 10 and 2 patches after 30 of context
+    blocks = [rows * 40, rows * (20 if kv_cache else 50), rows * (12 if kv_cache else 52)]
+    assert min(blocks[:2]) >= 768 and sum(blocks[:2]) >= 2048 and (blocks[2] < 768 + rows if kv_cache else True)
     got = _gpu(ta, m, x, obs, b, v, horizon, per_shot=per_shot, kv_cache=kv_cache)
     w8, w16 = (_oracle(o_, m, x, obs, b, v, horizon, 0, per_shot) for o_ in (orc, orc16))
     exact = _ref.timestral_forecast_f64(m, x, obs, b, v, horizon, per_shot=per_shot)
@@ -443,3 +443,40 @@ def test_timestral_weights_split_once_per_call(ta, orc, orc16, gpu_ready, b, v, 
     if not use_asinh:
         half = _gpu(ta, m, x, obs, b, v, horizon, per_shot=per_shot, kv_cache=kv_cache, attn_bf16=True)
         assert _ref.scaled_err(half, w16) < 1e-2
+
+
+@pytest.mark.parametrize("b,length,horizon,per_shot,kv_cache,kept", [
+    (1, 4000, 640, 8, False, False), (3, 6000, 512, 16, True, False), (3, 6000, 1024, 32, False, True)])
+def test_timestral_split_weights_are_held_only_where_blocks_read_them(ta, gpu_ready, b, length, horizon, per_shot,
+                                                                      kv_cache, kept):
+    """The copy of the layers' split weights is part of a forecast's scratch only if two of its decode blocks have
+    768 tokens and 2048 together: five blocks of 2 rows x (250 to 290) tokens, or one of 6 x 391 and a short one,
+    take none. By the device memory a first call in a fresh thread takes."""
+    import threading
+
+    import torch
+
+    rng = np.random.default_rng(b)
+    d, hid, layers = 512, 1536, 40
+    m = _ref.timestral_model(rng, d=d, nh=8, hid=hid, schedule=("variate",), context_length=1 << 20)
+    dm = _device_model(m)
+    dm["layers"] = dm["layers"] * layers
+    copy = layers * 6 * (5 * d * d + 3 * d * hid)  # three bf16 parts of every weight
+    x = torch.from_numpy(rng.standard_normal((b, length)).astype(np.float32)).cuda()
+    obs = torch.ones(b, length, device="cuda", dtype=torch.uint8)
+    out = torch.zeros(b, 1, horizon, m["q"], device="cuda")
+    taken = []
+
+    def call():
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        rc = ta.timestral_forecast(out, x, obs, dm, b, 1, length, horizon, per_shot=per_shot, kv_cache=kv_cache)
+        torch.cuda.synchronize()
+        taken.extend((rc, before - torch.cuda.mem_get_info()[0]))
+
+    t = threading.Thread(target=call)
+    t.start()
+    t.join()
+    assert taken[0] == ta.OK, ta.last_error()
+    # (Without the copy: activations and the products' workspaces, a third of it at most.)
+    assert taken[1] >= copy if kept else taken[1] < copy // 2, (taken, copy)

@@ -42,6 +42,11 @@ int main() {
                         if (s.shares > 1 && s.shares * blocks > most) most = s.shares * blocks;
                     }
             printf("%ld\n", most);
+        } else if (!strcmp(what, "keep")) {
+            KeptWeights k;
+            long tokens;
+            while (scanf("%ld", &tokens) == 1) k.add(tokens);
+            printf("%d\n", (int)k.pay());
         } else if (!strcmp(what, "big")) {
             long d_in, cus; int pre;
             if (scanf("%ld %d %ld", &d_in, &pre, &cus) != 3) return 1;
@@ -132,3 +137,11 @@ def test_shares_cover_the_reduction_and_fit_the_fixed_array(rules):
     tsfm_qkv_project_noalloc: at most 2 x 419 tiles of 64 x 64 floats, the figure in its header."""
     most = rules("splits")[0]
     assert most == 2 * 419 and most * 64 * 64 * 4 == 13729792 <= 16 << 20
+
+
+@pytest.mark.parametrize("blocks,keep", [
+    ([440, 94], 0), ([500] * 5, 0), ([1512, 564], 0), ([2016, 752], 0), ([1760, 376], 0), ([6512, 752], 0), ([2600], 0),
+    ([767] * 8, 0), ([768, 768, 432], 0), ([768, 768, 768, 432], 1), ([1900, 940], 1), ([3024, 1128], 1), ([1024, 1024], 1)])
+def test_split_weights_kept_for_a_forecast(rules, blocks, keep):
+    """Only blocks of 768 tokens read the kept copy, so only they count for it."""
+    assert rules("keep", *blocks) == [keep]

@@ -148,5 +148,24 @@ inline bool planes_pay(int64_t tokens, int64_t d_in, int64_t n_cols, bool whole,
     return macs >= (tokens < 1200 ? 18 : 15) * quarter;
 }
 
+// Whether a Timestral forecast splits its layers' weights once for all its decode blocks (a copy of 1.5x the
+// weights) instead of once per block and product. Only blocks of at least kKeptBlock tokens read the copy: shorter
+// ones split inside their products, whose reductions are shared out over more workgroups. It takes two such
+// blocks, of kKeptTokens together, to repay it. Whole forecasts, with the copy / without, four layers of 1024, by
+// the tokens of their blocks: 1520 and 752: 1.02, 1008, 512, 512 and 288: 1.02, 504 and 188: 1.10; three of
+// 768 and 432: 1.00; 1140, 768, 768 and 432: 0.98, 1900 and 940: 0.99, three of 1024 and 576: 0.97, 3024 and
+// 1128: 0.97.
+constexpr int64_t kKeptBlock = 768, kKeptTokens = 2048;
+struct KeptWeights {
+    int blocks = 0;
+    int64_t tokens = 0;
+    void add(int64_t block_tokens) {
+        if (block_tokens < kKeptBlock) return;
+        blocks++;
+        tokens += block_tokens;
+    }
+    bool pay() const { return blocks >= 2 && tokens >= kKeptTokens; }
+};
+
 }  // namespace rules
 }  // namespace tsfm

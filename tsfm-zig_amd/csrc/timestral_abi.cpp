@@ -29,6 +29,7 @@
 #include "../../include/tsfm_attn.h"
 #include "abi_internal.hpp"
 #include "launch.hpp"
+#include "rules.hpp"
 
 using tsfm::abi::aligned;
 using tsfm::abi::ensure_ready;
@@ -40,11 +41,7 @@ namespace {
 
 constexpr int kActSilu = 1;  // tsfm_resblock.act
 
-// The kept weight planes of a call: from this many tokens over all its blocks, up to this many bytes;
-// a block of fewer than kWeightPlanesBlock tokens splits inside its products instead, where the
-// reduction is shared out over more workgroups.
-constexpr int64_t kWeightPlanesTokens = 2048;
-constexpr int64_t kWeightPlanesBlock = 768;
+// The most bytes of weights a call splits once for all its blocks (rules::KeptWeights).
 constexpr size_t kWeightPlanesMax = (size_t)4 << 30;
 
 // One nn.linear (y = x w^T + bias) with an epilogue, over `rows` packed rows.
@@ -209,19 +206,16 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
     const int cap_tok = cap_p + per_shot + (cov ? per_shot : 0), sl_max = cap_tok;  // cov: window + decoder
     const int hpad = total_patches * ps;
     const bool cached = a->kv_cache != 0 && a->n_known == 0;
-    // Tokens of all decode blocks together, as the loop below runs them.
-    auto total_tokens = [&]() {
-        int64_t n = 0;
-        for (int left = total_patches, t = t_first, p0 = 0; left > 0;) {
-            const int h = std::min(per_shot, left), l = t / ps;
-            n += (int64_t)rows * ((cov ? l + h : l) - p0 + h);
-            left -= h;
-            const bool drop = t + h * ps > max_context;
-            p0 = drop || !cached ? 0 : l;
-            t = drop ? std::max(ps, max_context / ps * ps) : t + h * ps;
-        }
-        return n;
-    };
+    // The decode blocks, as the loop below runs them.
+    tsfm::rules::KeptWeights kept_blocks;
+    for (int left = total_patches, t = t_first, p0 = 0; left > 0;) {
+        const int h = std::min(per_shot, left), l = t / ps;
+        kept_blocks.add((int64_t)rows * ((cov ? l + h : l) - p0 + h));
+        left -= h;
+        const bool drop = t + h * ps > max_context;
+        p0 = drop || !cached ? 0 : l;
+        t = drop ? std::max(ps, max_context / ps * ps) : t + h * ps;
+    }
     if ((int64_t)rows * cap_tok * 3 * d > 0x7fffffffLL * 4) return fail(TSFM_E_UNSUPPORTED, "too large");
     hipStream_t s = static_cast<hipStream_t>(a->stream);
 
@@ -250,11 +244,9 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
     const size_t planes_n = tsfm::proj_plane_bytes((int64_t)rows * sl_max, std::max(d, hid), std::max(3 * d, 2 * hid));
     const size_t at_planes = plan.take(planes_n);
     // Pre-split operands (32-wide widths). at_xpl: the norms', gates' and MLP activations' results as the
-    // next product reads them. With several decode blocks, the layers' weights split once for the call (at_wpl)
-    // instead of once per block and product, when the blocks together are long enough to repay it and
+    // next product reads them. at_wpl: the layers' weights split once for the call, where its blocks repay it and
     // the copy (1.5x the weights) stays within kWeightPlanesMax.
     const bool splits = d % 32 == 0 && hid % 32 == 0;
-    const int64_t call_tokens = total_tokens();
     const size_t at_xpl = plan.take(splits ? tsfm::plane_operand_bytes((int64_t)rows * sl_max, std::max(d, hid)) : 0);
     size_t wpl_n = 0;
     for (int li = 0; li < M.n_layers; li++) {
@@ -262,8 +254,7 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
             wpl_n += tsfm::plane_operand_bytes((M.layers[li].attn[ai].gate ? 5 : 4) * (int64_t)d, d);
         wpl_n += tsfm::plane_operand_bytes(2 * (int64_t)hid, d) + tsfm::plane_operand_bytes(d, hid);
     }
-    const bool keep_weights = splits && total_patches > per_shot && call_tokens >= kWeightPlanesTokens &&
-                              wpl_n <= kWeightPlanesMax;
+    const bool keep_weights = splits && kept_blocks.pay() && wpl_n <= kWeightPlanesMax;
     const size_t at_wpl = plan.take(keep_weights ? wpl_n : 0);
     const size_t at_kf = plan.take((size_t)rows * hpad * 4 + 4), at_kfm = plan.take((size_t)rows * hpad + 1);
     const size_t at_noasinh = plan.take((size_t)rows);
@@ -385,7 +376,7 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
             const int toks = rows * sl;
             int ti = 0;
             // Which products of this block read their operands pre-split, and with kept weights.
-            const bool kept = keep_weights && toks >= kWeightPlanesBlock;
+            const bool kept = keep_weights && toks >= tsfm::rules::kKeptBlock;
             void* const XP = buf + at_xpl;
             const char* wp = buf + at_wpl;
             auto weights = [&](int64_t n, int64_t k) -> const void* {
