@@ -23,8 +23,9 @@
  *     gets its own HIP stream and device staging buffers, released when the thread exits; the
  *     device-pointer model calls keep their scratch per (thread, stream, entry point) between
  *     calls, released the same way;
- *   - results do not depend on how many host threads call in, nor on batch composition: there
- *     are no atomics in any reduction and tile order is fixed.
+ *   - results do not depend on how many host threads call in, nor on what the other rows of a
+ *     batch hold: there are no atomics in any reduction and tile order is fixed. How many rows a
+ *     call has picks its kernels, tiles and splits, and with them the last bits of f32 results.
  *
  * Layouts follow the reference: element (b, t, h, c) of Q lives at
  *   q[b * q_batch + t * q_tok + h * head_dim + c]
@@ -472,6 +473,10 @@ int tsfm_bolt_forecast_horizon(const tsfm_bolt_horizon_args *args);
  * scale when the model works in linear space. With use_asinh the head's outputs are sinh-expanded,
  * which turns bf16's relative rounding into a relative error of the forecast several times larger:
  * that combination returns TSFM_E_UNSUPPORTED.
+ * The scratch (activations, K/V caches, workspaces and, where two or more decode blocks are long enough to
+ * share them, the layers' weights split into bf16 parts: 1.5x their bytes, 4 GiB at most) is kept for the
+ * calling thread and stream between calls, as large as the largest call needed. A device without room for
+ * the split weights, or for the split activations beside them, runs the forecast without.
  * Errors as the reference's: covariates with covariate_enabled == 0 (error.CovariatesUnsupported),
  * known covariates with a schedule that cannot route them (error.KnownCovariatesUnsupported) return
  * TSFM_E_UNSUPPORTED; a covariate array with a zero count, or a count without its array, returns

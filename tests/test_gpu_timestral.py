@@ -480,3 +480,57 @@ def test_timestral_split_weights_are_held_only_where_blocks_read_them(ta, gpu_re
     assert taken[0] == ta.OK, ta.last_error()
     # (Without the copy: activations and the products' workspaces, a third of it at most.)
     assert taken[1] >= copy if kept else taken[1] < copy // 2, (taken, copy)
+
+
+_ONE_FORECAST = """
+import sys
+import numpy as np, torch
+import tsfm_attn as ta
+import _ref
+from test_gpu_timestral import _device_model
+out_path, layers = sys.argv[1], int(sys.argv[2])
+try:
+    torch.empty(4 << 30, dtype=torch.uint8, device="cuda")
+    bounded = 0
+except torch.cuda.OutOfMemoryError:
+    bounded = 1
+rng = np.random.default_rng(7)
+m = _ref.timestral_model(rng, d=512, nh=8, hid=1536, schedule=("variate",), context_length=1 << 20)
+dm = _device_model(m)
+dm["layers"] = dm["layers"] * layers
+b, length, horizon = 3, 3000, 1024
+x = torch.from_numpy(rng.standard_normal((b, length)).astype(np.float32)).cuda()
+obs = torch.ones(b, length, device="cuda", dtype=torch.uint8)
+out = torch.zeros(b, 1, horizon, m["q"], device="cuda")
+for _ in range(2):
+    rc = ta.timestral_forecast(out, x, obs, dm, b, 1, length, horizon, per_shot=32, kv_cache=False)
+    assert rc == ta.OK, ta.last_error()
+torch.cuda.synchronize()
+np.savez(out_path, out=out.cpu().numpy(), bounded=bounded)
+"""
+
+
+def test_timestral_forecast_without_room_for_the_split_weights(ta, gpu_ready, tmp_path):
+    """A forecast whose scratch fits the device without the copy of the split weights (here 3.1 GB), but not with it,
+    runs without. The runtime bounds single allocations to 1 % of the memory in one of two processes."""
+    import os
+    import pathlib
+    import subprocess
+    import sys
+
+    here = pathlib.Path(__file__).resolve().parent
+    outs = []
+    for percent in (None, "1"):
+        env = dict(os.environ, PYTHONPATH=os.pathsep.join([str(here.parent / "tsfm-zig_amd"), str(here)]))
+        if percent:
+            env["GPU_SINGLE_ALLOC_PERCENT"] = percent
+        path = tmp_path / f"out{percent}.npz"
+        run = subprocess.run([sys.executable, "-c", _ONE_FORECAST, str(path), "140"], env=env, capture_output=True,
+                             text=True, timeout=100)
+        assert run.returncode == 0, run.stdout + run.stderr
+        with np.load(path) as z:
+            outs.append((z["out"], int(z["bounded"])))
+    if not outs[1][1] or outs[0][1]:
+        pytest.skip("the runtime does not bound single allocations here")
+    assert np.isfinite(outs[0][0]).all()
+    assert _ref.scaled_err(outs[1][0], outs[0][0]) < 2e-5

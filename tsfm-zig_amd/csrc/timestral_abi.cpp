@@ -243,24 +243,40 @@ extern "C" int tsfm_timestral_forecast(const tsfm_timestral_forecast_args* a) {
     const size_t at_part = plan.take(tsfm::kSplitWorkspaceBytes);
     const size_t planes_n = tsfm::proj_plane_bytes((int64_t)rows * sl_max, std::max(d, hid), std::max(3 * d, 2 * hid));
     const size_t at_planes = plan.take(planes_n);
-    // Pre-split operands (32-wide widths). at_xpl: the norms', gates' and MLP activations' results as the
-    // next product reads them. at_wpl: the layers' weights split once for the call, where its blocks repay it and
-    // the copy (1.5x the weights) stays within kWeightPlanesMax.
-    const bool splits = d % 32 == 0 && hid % 32 == 0;
+    const size_t at_kf = plan.take((size_t)rows * hpad * 4 + 4), at_kfm = plan.take((size_t)rows * hpad + 1);
+    const size_t at_noasinh = plan.take((size_t)rows);
+    // What only saves time, last: a device without room for it runs the forecast without. Pre-split operands
+    // (32-wide widths): at_xpl, the norms', gates' and MLP activations' results as the next product reads them;
+    // at_wpl, the layers' weights split once for the call, where its blocks repay it and the copy (1.5x the
+    // weights) stays within kWeightPlanesMax.
+    bool splits = d % 32 == 0 && hid % 32 == 0;
+    const size_t need = plan.off;
     const size_t at_xpl = plan.take(splits ? tsfm::plane_operand_bytes((int64_t)rows * sl_max, std::max(d, hid)) : 0);
+    const size_t with_operands = plan.off;
     size_t wpl_n = 0;
     for (int li = 0; li < M.n_layers; li++) {
         for (int ai = 0; ai < M.layers[li].n_attn; ai++)
             wpl_n += tsfm::plane_operand_bytes((M.layers[li].attn[ai].gate ? 5 : 4) * (int64_t)d, d);
         wpl_n += tsfm::plane_operand_bytes(2 * (int64_t)hid, d) + tsfm::plane_operand_bytes(d, hid);
     }
-    const bool keep_weights = splits && kept_blocks.pay() && wpl_n <= kWeightPlanesMax;
+    bool keep_weights = splits && kept_blocks.pay() && wpl_n <= kWeightPlanesMax;
     const size_t at_wpl = plan.take(keep_weights ? wpl_n : 0);
-    const size_t at_kf = plan.take((size_t)rows * hpad * 4 + 4), at_kfm = plan.take((size_t)rows * hpad + 1);
-    const size_t at_noasinh = plan.take((size_t)rows);
     char* buf = nullptr;
     bool owned = false;
-    hipError_t e = tsfm::abi::scratch_acquire(s, tsfm::abi::kSlotTimestralForecast, plan.off, &buf, &owned);
+    auto acquire = [&](size_t bytes) {
+        return tsfm::abi::scratch_acquire(s, tsfm::abi::kSlotTimestralForecast, bytes, &buf, &owned);
+    };
+    hipError_t e = acquire(plan.off);
+    if (e == hipErrorOutOfMemory && keep_weights) {
+        (void)hipGetLastError();  // (else the next launch would report it)
+        keep_weights = false;
+        e = acquire(with_operands);
+    }
+    if (e == hipErrorOutOfMemory && splits) {
+        (void)hipGetLastError();
+        splits = false;
+        e = acquire(need);
+    }
     if (e != hipSuccess) return hip_fail(e, "forecast scratch allocation");
     auto F = [&](size_t at) { return reinterpret_cast<float*>(buf + at); };
     auto U8 = [&](size_t at) { return reinterpret_cast<uint8_t*>(buf + at); };
