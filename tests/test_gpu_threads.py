@@ -183,3 +183,41 @@ def test_fused_row_norm_equals_the_separate_launch(ta, gpu_ready):
     finally:
         del os.environ["TSFM_UNFUSED_NORM"]
     assert np.array_equal(fused, separate)
+
+
+@pytest.mark.parametrize("b,seq,nh,d_ff", [(5, 109, 12, 3072), (2, 8, 12, 3072), (3, 100, 2, 192), (16, 131, 12, 3072)])
+def test_encoder_row_norms_with_the_products_equal_the_separate_launches(ta, gpu_ready, b, seq, nh, d_ff):
+    """The Chronos-2 encoder hands each residual product the row norm after it, the last one in place: 545 rows
+    (the products split their reduction and the reduce normalises), 16 (the 16-row products), 300 of 128 values
+    (unsplit: a launch of its own), 2096 (pre-split operands). The same bits as separate launches
+    (TSFM_UNFUSED_NORM=1)."""
+    import os
+
+    import torch
+
+    import _ref
+
+    rng = np.random.default_rng(b * seq)
+    d, eps = nh * 64, 1e-6
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    x = rng.standard_normal((b * seq, d)).astype(np.float32)
+    kv = cu(_ref.left_pad_valid(rng, b, seq, seq // 4, tail_valid=2))
+    layers = [{k: cu(v) for k, v in ly.items()} for ly in _ref.chronos2_layers(rng, 2, d, d_ff)]
+    fn = cu((1 + 0.1 * rng.standard_normal(d)).astype(np.float32))
+    ang = np.outer(np.arange(seq), 10000.0 ** (-np.arange(32) / 32))
+    cs, sn = cu(np.cos(ang).astype(np.float32)), cu(np.sin(ang).astype(np.float32))
+
+    def run():
+        y = cu(x)
+        rc = ta.chronos2_encode(y, kv, cs, sn, layers, fn, b, seq, d, nh, d_ff, eps, keys_all_valid=False)
+        assert rc == ta.OK, ta.last_error()
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    fused = run()
+    os.environ["TSFM_UNFUSED_NORM"] = "1"
+    try:
+        separate = run()
+    finally:
+        del os.environ["TSFM_UNFUSED_NORM"]
+    assert np.isfinite(fused).all() and np.array_equal(fused, separate)
