@@ -1,5 +1,6 @@
-// f32 attention for short rows (n_k <= 144: Chronos-Bolt's 129-token rows), on the f32 matrix
-// cores (v_mfma_f32_16x16x4_f32). Longer rows take the bf16x3 streaming kernel (attn_x3.hip).
+// f32 attention for short rows (n_k <= 144) on the f32 matrix cores (v_mfma_f32_16x16x4_f32): few rows of few
+// queries, most rows of 32k + 1, the causal masks, single queries (rules::attn_x3_pays). Longer rows, and the
+// other short ones, take the bf16x3 kernel (attn_x3.hip).
 //
 // The reference computes one (series, head) at a time with a materialised n x n score matrix:
 // gemmNT -> bias -> masked softmax -> gemmNN (src/core/attn.zig:72-96). Here the whole batch is one
@@ -96,7 +97,7 @@ __device__ __forceinline__ void load_q(QBlock& w, const float* Q, const float* R
 // is below n_k and valid, every query past it for the causal masks, so the body has no bounds tests
 // and no mask arithmetic; otherwise only the first nkb key blocks are computed and every score goes
 // through the mask rule. hook(phase, kb) runs at fixed points (S block kb, after S, PV block kb)
-// whether or not the block is computed: the streaming kernel stages the next tile there.
+// whether or not the block is computed: work that can run between the matrix instructions goes there.
 // VROW: vt holds V as rows [key][64] and the O^T accumulator takes the dims in the order
 // 16g + 4r + db (register r of w.o[db]): the V operands of one key for the four dim blocks are then
 // four consecutive floats of its row (the bits of O are the same; only its register order moves).
@@ -405,14 +406,11 @@ __device__ __forceinline__ void store_o(const QBlock& w, float* O, const Params&
 
 // ---- short rows: every key resident in LDS ------------------------------------------------------
 //
-// Chronos-Bolt rows are short (at most 128 patches + REG = 129 tokens). Streamed through the
-// two-stage pipeline above they pay a staging round and a barrier for each of three tiles, and
-// 128-query workgroups leave a one-query tail workgroup (129 = 128 + 1) that stages all of K/V
-// again. Here one workgroup of 9 waves (one 16-query block each, 144 queries) loads the whole K, V,
-// key terms and T5 table of its (series, head) into LDS once; then every wave runs the per-tile
-// arithmetic above over the resident keys with no further barrier. The waves of a workgroup land
-// two or three to a SIMD, so two workgroups per CU need room for six waves per SIMD: the kernel is
-// built for 80 VGPRs (a few spill to scratch; no global load is in flight there).
+// One workgroup of 9 waves (one 16-query block each, 144 queries: 129 tokens in one workgroup) loads the
+// whole K, V, key terms and T5 table of its (series, head) into LDS once; then every wave runs the
+// per-tile arithmetic above over the resident keys with no further barrier. One workgroup a CU takes
+// the rows in turn, the next row's operands on their way into a second buffer meanwhile; its waves land
+// two or three to a SIMD, and the kernel is built for three.
 
 constexpr int RNW = 9;                  // waves per workgroup
 constexpr int RNT = 64 * RNW;           // threads

@@ -8,7 +8,7 @@
 // time of sixteen, and with the VALU free to run the softmax beside it (the f32 matrix instruction
 // and the VALU never overlap on this part; the bf16 one does).
 //
-// One workgroup = one (series, head) x nw query blocks of 32 (nw waves, 4 to 8), on
+// One workgroup = one (series, head) x nw query blocks of 32 (nw = 4 waves), on
 // v_mfma_f32_32x32x16_bf16. Per 32-key chunk and wave:
 //   S^T = K . Q^T   A = K (lane: key l%32, dims 16s + 8(l/32)..+7), B = Q^T from registers (lane:
 //                   query l%32, same dims), four k-steps over the 64 head dims. The five small
@@ -89,8 +89,8 @@ __device__ __forceinline__ void split4(f32x4 v, u32x2& hi, u32x2& mid, u32x2& lo
     mid = u32x2{a.m, b.m};
     lo = u32x2{a.l, b.l};
 }
-// 1 for a row of 32k + 1 queries that one workgroup takes (1 <= k <= 8): its last query runs
-// outside the 32-query blocks, at the end of the workgroup, instead of as a 32-query block of its own
+// 1 for a row of 32k + 1 queries that one workgroup takes (1 <= k <= 4): its last query runs
+// outside the 32-query blocks, at the start of the workgroup, instead of as a 32-query block of its own
 // (longer rows keep that block: there the pass would lengthen one workgroup in three).
 __host__ __device__ inline int thin_query(int n_q) { return (n_q > XQ && n_q <= XMAXW * XQ + 1 && n_q % XQ == 1) ? 1 : 0; }
 

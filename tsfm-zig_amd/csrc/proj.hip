@@ -891,20 +891,22 @@ __global__ __launch_bounds__(256) void proj_reduce_norm(ProjParams p) {
 // RoPE. Such a product is a few MB of weights read once: it is bound by how many loads are in
 // flight, not by the matrix cores. A workgroup takes one 16-column tile of every token and its
 // sixteen waves split the reduction: wave w takes the 16-wide units [w U / 16, (w + 1) U / 16) of
-// U = d_in / 16 and issues the loads of SKB of them at once, straight from HBM/L2 into
-// registers in the matrix instruction's layout (lane l: row l & 15 of a 16-row block, indices
-// 4 (l >> 4) .. + 3 of the unit), then multiplies them, accumulating blockwise as qkv_proj does.
+// U = d_in / 16, SKB at a time: their loads go straight from HBM/L2 into registers in the matrix
+// instruction's layout (lane l: row l & 15 of a 16-row block, indices 4 (l >> 4) .. + 3 of the unit), then
+// it multiplies them, accumulating blockwise as qkv_proj does, and the next batch's loads follow (two
+// batches at 1024 indices, four at 2048, one behind the other: other waves cover their waits).
 // The sixteen 16 x 16 partials meet in LDS and are added in wave order, then the epilogue: one
 // launch where a split over workgroups would need a second one for the sums.
 constexpr int SKW = 16;  // waves of a workgroup
-constexpr int SKB = 2;   // units in a batch: a 1024-thread workgroup has 128 registers a lane, and eight
-                         // units with the norm's row in flight too spilled 32 of them
+constexpr int SKB = 2;   // units in a batch: a 1024-thread workgroup has 128 registers a lane (70 used), and
+                         // eight units with the norm's row in flight too spilled 32 of them
 constexpr int kSkinnyTokens = 16;
 // The longest reductions it takes, and with the input norm (the norm's row is held in registers).
 // Longer ones read more weight bytes per column tile than the few CUs of the launch pull in time and
 // split over workgroups instead, whose sum costs a second launch. Whole Chronos-Bolt forecasts in us,
 // longest 1024 / 2048 / 3072: 16 series of d_ff 2048 917 / 908 / 918, of 3072 883 / 874 / 886; 4 series of
-// 3072 661 / 654 / 635, one 482 / 469 / 432, one of d_ff 2048 376 / 348 / 348.
+// 3072 661 / 654 / 635, one 482 / 469 / 432, one of d_ff 2048 376 / 348 / 348 (no reductions in between
+// were measured).
 constexpr int kSkinnyNormIn = 1024;
 static int skinny_max_in(int64_t tokens) { return tokens <= 8 ? 3072 : 2048; }
 constexpr size_t kSkinnyLds = (size_t)SKW * kSkinnyTokens * 16 * sizeof(float);

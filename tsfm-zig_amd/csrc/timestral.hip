@@ -324,8 +324,10 @@ __global__ __launch_bounds__(kStatsT) void ts_stats(const TsStatsParams p) {
             st_s[0] = cw[n - 1];
         } else if (tid == 64) {
             // welfordCombine (forecaster.zig:567-577), its mean: a division by the running count w per
-            // patch. a / w from y = 1 / w (rounded): q = a y, then q + (a - w q) y is the rounded
-            // quotient (Markstein's theorem); values past its range divide.
+            // patch. a / w from y = 1 / w (rounded): q = a y is off by 1.5 ulp at most, a - w q is then
+            // exact, and q + (a - w q) y lies within 2^-51 ulp of a / w before it is rounded. It rounds as a / w
+            // does because w is a whole number: a / w is at least 1 / (2 w) ulp away from the middle of two
+            // doubles. Values past the range of the products divide.
             double fw = fold_w0, fmean = fo_s[1];
 #pragma unroll 4
             for (int q = 0; q < np; q++) {
