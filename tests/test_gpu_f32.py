@@ -428,8 +428,8 @@ def test_short_rows_on_both_sides_of_the_kernel_choice(ta, gpu_ready, mask, n_q,
 def test_short_rows_with_infinite_and_huge_operands(ta, gpu_ready, mask, n_q, n_k, form):
     """Rows of at most 144 keys give what f32 arithmetic gives on either kernel: an infinite K value
     whose scores are all -inf leaves its key without weight, as a finite one past the largest bf16 (3.39e38)
-    does; such a V value gives finite outputs, an infinite one an infinite dim and no other. 516 rows of
-    one size, and 2."""
+    does; such a V value gives finite outputs, an infinite one an infinite dim and no other, NaN likewise; a
+    NaN in K every output of its head. 516 rows of one size, and 2."""
     rng = np.random.default_rng(n_q + 1000 * mask)
     H = 6
     extra = dict(q_pos0=n_k - n_q) if mask >= 2 else {}
@@ -451,7 +451,7 @@ def test_short_rows_with_infinite_and_huge_operands(ta, gpu_ready, mask, n_q, n_
         cos_t, sin_t = np.cos(ang).astype(np.float32), np.sin(ang).astype(np.float32)
         extra.update(rope_cos=cos_t, rope_sin=sin_t)
     key = 0 if mask in (2, 5) else n_k - 1 if n_k % 32 == 1 else n_k // 2
-    for kind in ("v_inf", "v_huge") + (() if form == "rope" else ("k_inf", "k_huge")):
+    for kind in ("v_inf", "v_huge", "v_nan", "k_nan") + (() if form == "rope" else ("k_inf", "k_huge")):
         for B in (86, 1):
             heads = H if B > 1 else 2
             q, k, v, kv = _inputs(n_q + B, B, heads, n_q, n_k)
@@ -459,7 +459,7 @@ def test_short_rows_with_infinite_and_huge_operands(ta, gpu_ready, mask, n_q, n_
             kv[:, key] = 1
             if kind[0] == "k":
                 q[:, :, ::64] = 1.0
-            bad = dict(v_inf=np.inf, v_huge=3.4e38, k_inf=-np.inf, k_huge=-3.4e38)[kind]
+            bad = dict(v_inf=np.inf, v_huge=3.4e38, k_inf=-np.inf, k_huge=-3.4e38).get(kind, np.nan)
             (k if kind[0] == "k" else v)[:, key, ::64] = bad
             got = run_generic(ta, mask, q, k, v, kv, B, heads, n_q, n_k, 1.0,
                               **{n: a[:heads] if n == "bias" else np.ascontiguousarray(a[:, :heads]) if n == "rel_table" else a

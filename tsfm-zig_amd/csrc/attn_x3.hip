@@ -108,18 +108,44 @@ __device__ __forceinline__ float pair_sum(float x) {
 // a value that rounds past the largest bf16 (inf - inf), so such an operand makes the row's scores or
 // outputs NaN where f32 arithmetic may not: a score of -inf has weight 0, an infinite V gives infinite
 // outputs. Same bias, mask and weights as the resident f32 kernel, which other calls of such rows run on;
-// the keys it weighs with 0 past the query's own range (whole 16-key blocks) included. scr: kRedoScratch
-// floats of the wave's own. Only the check runs when the results are finite: 32 additions a wave (256 x 12
-// rows of 129 with the T5 bias: 142.4 us with it, 142.0 without).
+// the keys it weighs with 0 past the query's own range (whole 16-key blocks) included. False, and the
+// result stands, when no operand is that large (kv_huge: some K or V value is): then only a NaN among
+// them makes it NaN, as in f32. scr: kRedoScratch floats of the wave's own. Only the check runs when the
+// results are finite: 32 additions a wave (256 x 12 rows of 129 with the T5 bias: 140.4 us with it, 139.4
+// without). With every K value NaN that launch takes 245 us, and 3229 if each query were computed again.
 constexpr int kRedoScratch = kHeadDim + (kResidentKeys + 63) / 64 * 64;
-template <int MASK, int BIAS, bool ROPE>
-__device__ __forceinline__ float redo_query(const float* lut, float* scr, int b, int h, int qi, int lane) {
-#pragma clang fp contract(off)
-    // The kernel's arguments read again, through a pointer the optimiser cannot see through: kept from the
-    // top of the kernel for this path, they would take up to thirty scalar registers through its loops.
+__device__ __forceinline__ bool huge(float x) { return fabsf(x) >= 1e18f; }  // (products of two such still fit f32)
+
+// The kernel's arguments read again, through a pointer the optimiser cannot see through: kept from the
+// top of the kernel for the cold paths below, they would take up to thirty scalar registers through its loops.
+__device__ __forceinline__ const Params& reread_params() {
     uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(args));
-    const Params& p = *(const Params*)(const __attribute__((address_space(4))) Params*)args;
+    return *(const Params*)(const __attribute__((address_space(4))) Params*)args;
+}
+
+// Whether a K or V value of the (series, head) is huge (K as given: a rotation by cosines and sines adds no more
+// than half to it). Four keys at a time, sixteen bytes a lane. The loops of the cold path stay rolled: unrolled
+// ones cost the kernel's own loop registers.
+__device__ __forceinline__ bool any_huge(int b, int h, int lane) {
+    const Params& p = reread_params();
+    const float* const K = static_cast<const float*>(p.k) + b * p.k_batch + h * kHeadDim + 4 * (lane & 15);
+    const float* const V = static_cast<const float*>(p.v) + b * p.v_batch + h * kHeadDim + 4 * (lane & 15);
+    float most = 0.f;  // (fmaxf takes the other operand of a NaN)
+#pragma unroll 1
+    for (int key = lane >> 4; key < p.n_k; key += 4) {
+        const f32x4 kk = ld4(K + (int64_t)key * p.k_tok), vv = ld4(V + (int64_t)key * p.v_tok);
+#pragma unroll
+        for (int i = 0; i < 4; i++) most = fmaxf(most, fmaxf(fabsf(kk[i]), fabsf(vv[i])));
+    }
+    return __ballot(huge(most)) != 0;
+}
+
+template <int MASK, int BIAS, bool ROPE>
+__device__ __forceinline__ bool redo_query(float& out, const float* lut, float* scr, bool kv_huge, int b, int h, int qi,
+                                           int lane) {
+#pragma clang fp contract(off)
+    const Params& p = reread_params();
     const float* const Q = static_cast<const float*>(p.q) + b * p.q_batch + h * kHeadDim;
     const float* const K = static_cast<const float*>(p.k) + b * p.k_batch + h * kHeadDim;
     const float* const V = static_cast<const float*>(p.v) + b * p.v_batch + h * kHeadDim;
@@ -130,17 +156,17 @@ __device__ __forceinline__ float redo_query(const float* lut, float* scr, int b,
     const int qpos = p.q_pos0 + qi;
     const int kend =
         min(p.n_k, (key_end_for<MASK>(p.q_pos0 + min(p.n_q - 1, qi | 15), p.n_k, p.ctx_keys) + 15) & ~15);
-    if (lane < 32) {
-        float x1 = Q[(int64_t)qi * p.q_tok + lane], x2 = Q[(int64_t)qi * p.q_tok + lane + 32];
-        if (ROPE) {  // nn.ropeHalf, src/core/nn.zig:453-460
-            const float c = RC[(int64_t)qpos * 32 + lane], sn = RS[(int64_t)qpos * 32 + lane];
-            const float y1 = x1 * c - x2 * sn, y2 = x2 * c + x1 * sn;
-            x1 = y1;
-            x2 = y2;
-        }
-        scr[lane] = x1 * p.scale;
-        scr[lane + 32] = x2 * p.scale;
+    float x1 = Q[(int64_t)qi * p.q_tok + (lane & 31)], x2 = Q[(int64_t)qi * p.q_tok + (lane & 31) + 32];
+    if (ROPE) {  // nn.ropeHalf, src/core/nn.zig:453-460
+        const float c = RC[(int64_t)qpos * 32 + (lane & 31)], sn = RS[(int64_t)qpos * 32 + (lane & 31)];
+        const float y1 = x1 * c - x2 * sn, y2 = x2 * c + x1 * sn;
+        x1 = y1;
+        x2 = y2;
     }
+    x1 = x1 * p.scale;
+    x2 = x2 * p.scale;
+    if (!kv_huge && __ballot(huge(x1) || huge(x2)) == 0) return false;
+    scr[lane] = lane < 32 ? x1 : x2;
     __builtin_amdgcn_wave_barrier();  // LDS keeps a wave's accesses in order
     float* const w = scr + kHeadDim;
     float m = kNegInf;
@@ -175,10 +201,11 @@ __device__ __forceinline__ float redo_query(const float* lut, float* scr, int b,
     }
     for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
     __builtin_amdgcn_wave_barrier();
-    float out = 0.f;
-#pragma unroll 4
-    for (int key = 0; key < kend; key++) out = __builtin_fmaf(w[key], V[(int64_t)key * p.v_tok + lane], out);
-    return out * (1.0f / l);
+    float acc = 0.f;
+#pragma unroll 1
+    for (int key = 0; key < kend; key++) acc = __builtin_fmaf(w[key], V[(int64_t)key * p.v_tok + lane], acc);
+    out = acc * (1.0f / l);
+    return true;
 }
 
 // SHORT: rows of at most kResidentKeys keys, whose results are checked (redo_query). A kernel of its own:
@@ -668,10 +695,12 @@ __global__ __launch_bounds__(XNT) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
             const float sum = (part[0] + part[1]) + (part[2] + part[3]);
             const uint64_t odd = __ballot(ql < wave_nq && !(fabsf(sum) <= kFltMax));
             uint64_t todo = ((odd | odd >> 32) & 0xffffffffu) | (uint64_t)thin_odd << 32;  // bit 32: the single query
+            const bool kv_huge = todo != 0 && any_huge(b, h, lane);
             for (; todo != 0; todo &= todo - 1) {
                 const int r = __builtin_ctzll(todo), q = r < XQ ? wq0 + r : p.n_q - 1;
                 float* const scr = reinterpret_cast<float*>(&stage[0]) + XMAXW * XQ * kHeadDim + wave * kRedoScratch;
-                const float y = redo_query<MASK, BIAS, ROPE>(lut, scr, b, h, q, lane);
+                float y;
+                if (!redo_query<MASK, BIAS, ROPE>(y, lut, scr, kv_huge, b, h, q, lane)) continue;
                 if (r < XQ) ob[r * kHeadDim + 4 * ((lane >> 2) ^ (r & 15)) + (lane & 3)] = y;
                 else O[(int64_t)q * p.o_tok + lane] = y;
             }
