@@ -111,8 +111,8 @@ __device__ __forceinline__ float pair_sum(float x) {
 // the keys it weighs with 0 past the query's own range (whole 16-key blocks) included. False, and the
 // result stands, when no operand is that large (kv_huge: some K or V value is): then only a NaN among
 // them makes it NaN, as in f32. scr: kRedoScratch floats of the wave's own. Only the check runs when the
-// results are finite: 32 additions a wave (256 x 12 rows of 129 with the T5 bias: 140.4 us with it, 139.4
-// without). With every K value NaN that launch takes 245 us, and 3229 if each query were computed again.
+// results are finite: sixteen maxima a wave (256 x 12 rows of 129 with the T5 bias: 143.0 us with it, 142.1
+// without; 32 additions in their place 143.7). With every K value NaN that launch takes 245 us, and 3229 if each query were computed again.
 constexpr int kRedoScratch = kHeadDim + (kResidentKeys + 63) / 64 * 64;
 __device__ __forceinline__ bool huge(float x) { return fabsf(x) >= 1e18f; }  // (products of two such still fit f32)
 
@@ -688,12 +688,13 @@ __global__ __launch_bounds__(XNT) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
                     f32x4{o[db][4 * g4], o[db][4 * g4 + 1], o[db][4 * g4 + 2], o[db][4 * g4 + 3]} * inv;
             }
         if constexpr (SHORT) {
-            // Not finite if a value of the lane's is not (or if the sum of finite ones overflows: redone alike).
-            f32x4 part = {0.f, 0.f, 0.f, 0.f};
+            // The largest magnitude of the lane's values, or NaN (gfx950's three-operand maximum passes NaN on).
+            float most = 0.f;
 #pragma unroll
-            for (int r = 0; r < 32; r++) part[r & 3] += o[r >> 4][r & 15];
-            const float sum = (part[0] + part[1]) + (part[2] + part[3]);
-            const uint64_t odd = __ballot(ql < wave_nq && !(fabsf(sum) <= kFltMax));
+            for (int r = 0; r < 32; r += 2)
+                most = __builtin_elementwise_maximum(
+                    __builtin_elementwise_maximum(fabsf(o[r >> 4][r & 15]), fabsf(o[r >> 4][(r & 15) + 1])), most);
+            const uint64_t odd = __ballot(ql < wave_nq && !(most <= kFltMax));
             uint64_t todo = ((odd | odd >> 32) & 0xffffffffu) | (uint64_t)thin_odd << 32;  // bit 32: the single query
             const bool kv_huge = todo != 0 && any_huge(b, h, lane);
             for (; todo != 0; todo &= todo - 1) {
